@@ -1358,7 +1358,14 @@ static hipError_t enqueue_step(rstr_decoder* d, hipStream_t st, Prof* prof, bool
                       w == 1 ? md.sliding_window : 0, md.attn_scale};
   }
   const size_t tabw = d->tabw;
-  run(RSTR_K_ROWS, [&] { return launch_attn_lists(st, geo, has_window ? 2 : 1, len, d->lane_tab, tabw, d->max_items); });
+  // a prefill tile's rows share one route: the tile kernel reads the lane tables, not the work list
+  const bool tile = !d->head_tail && attn_tiles(geo[0]);
+  if (tile) {
+    for (int w = 0; w < (has_window ? 2 : 1); w++)
+      run(RSTR_K_ROWS, [&] { return launch_attn_tables(st, geo[w], len, d->lane_tab + w * tabw, d->max_items); });
+  } else {
+    run(RSTR_K_ROWS, [&] { return launch_attn_lists(st, geo, has_window ? 2 : 1, len, d->lane_tab, tabw, d->max_items); });
+  }
   run(RSTR_K_ROWS, [&] {
     return launch_rms_quant(st, d->r0, d->m->layers[0].attn_norm, goff, md.eps, B, dm, d->act);
   });
@@ -1390,6 +1397,7 @@ static hipError_t enqueue_step(rstr_decoder* d, hipStream_t st, Prof* prof, bool
                                md.eps, cos_l, sin_l, pos, slots, d->qr, kp, vp);
       });
       run(RSTR_K_ATTN_SPLIT, [&] {
+        if (tile) return launch_attn_tile(st, geo[wi], d->qr, kp, vp, pt, len, d->lane_tab + wi * tabw, d->part);
         return launch_attn_split(st, geo[wi], d->qr, kp, vp, pt, d->lane_tab + wi * tabw, d->part, d->max_items,
                                  d->attn_direct ? &aout : nullptr);
       });
