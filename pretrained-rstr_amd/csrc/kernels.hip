@@ -2460,314 +2460,395 @@ __global__ __launch_bounds__(64) void k_attn_split(
 }
 
 // ---- qkv post-processing inside the few-item kernel (AttnQkv) --------------------
-// One head of row `src`'s qkv output with k_qkv_post's arithmetic: lane l <
-// HD/4 holds elements 4l..4l+3 (slices added in the canonical tree), then the
-// optional RMS norm over the head.
+// One head of a row's qkv output with k_qkv_post's arithmetic: lane l < HD/4
+// holds elements 4l..4l+3 (slices added in the canonical tree).  The optional
+// RMS norm over the head:
 template <int HD>
-__device__ __forceinline__ f4 qkv_head(const AttnQkv& qk, size_t src, const float* gn, int lane) {
-  constexpr int HD4 = HD / 4;
-  const bool have = lane < HD4;
-  const int cc = have ? lane : 0;
-  f4 v;
-  if (qk.y.n == 1) v = sl_get<1>(qk.y, src + 4 * cc);
-  else if (qk.y.n == 2) v = sl_get<2>(qk.y, src + 4 * cc);
-  else v = sl_get<4>(qk.y, src + 4 * cc);
-  if (gn) {
-    const f4 gg = *reinterpret_cast<const f4*>(gn + 4 * cc);
-    float a = 0.0f;
-    if (have) {
-      a = __builtin_fmaf(v[0], v[0], a);
-      a = __builtin_fmaf(v[1], v[1], a);
-      a = __builtin_fmaf(v[2], v[2], a);
-      a = __builtin_fmaf(v[3], v[3], a);
-    }
-    // HD/4 <= 64 chunks: lane l holds slot l alone, and the tree over 64
-    // lanes equals the 256-slot tree (the other slots are +0)
-    const float r = rms_scale(wave_tree_sum(a), HD, qk.eps);
-#pragma unroll
-    for (int i = 0; i < 4; i++) v[i] = (v[i] * r) * (qk.goff + gg[i]);
+__device__ __forceinline__ f4 qkv_norm(const AttnQkv& qk, f4 v, f4 gg, int lane) {
+  float a = 0.0f;
+  if (lane < HD / 4) {
+    a = __builtin_fmaf(v[0], v[0], a);
+    a = __builtin_fmaf(v[1], v[1], a);
+    a = __builtin_fmaf(v[2], v[2], a);
+    a = __builtin_fmaf(v[3], v[3], a);
   }
+  // HD/4 <= 64 chunks: lane l holds slot l alone, and the tree over 64
+  // lanes equals the 256-slot tree (the other slots are +0)
+  const float r = rms_scale(wave_tree_sum(a), HD, qk.eps);
+#pragma unroll
+  for (int i = 0; i < 4; i++) v[i] = (v[i] * r) * (qk.goff + gg[i]);
   return v;
 }
-
-// The item's q heads (wave w: heads w, w+4, ...) into qst[G][HD], rotated at the
-// row's position; the item holding the lane's newest token also writes that
-// token's K (wave 0: norm, RoPE) and V (wave 1) to the pages at the slot.
-// Every write is complete and visible to the workgroup on return.
-template <int HD, int G>
-__device__ void attn_qkv_prologue(const AttnQkv& qk, const AttnItem& it, int n_kv, int lane, int wave,
-                                  float* qst) {
-  constexpr int HD4 = HD / 4, HALF = HD / 2;
-  const int kvr = n_kv * HD, qd = n_kv * G * HD;
-  const size_t yr = (size_t)it.b * (qd + 2 * kvr);
-  const bool have = lane < HD4;
-  const int slot = uni(qk.slots[it.b]);
-  const bool newest = slot >= 0 && it.t1 == uni(qk.lengths[it.b]);
-  const int pos = uni(qk.positions[it.b]);
-  float* kst = qst + G * HD;
-  for (int h = wave; h < G; h += 4) {
-    const f4 v = qkv_head<HD>(qk, yr + (size_t)(it.kvh * G + h) * HD, qk.qn, lane);
-    if (have) *reinterpret_cast<f4*>(qst + h * HD + 4 * lane) = v;
-  }
-  if (newest && wave == 0) {
-    const f4 v = qkv_head<HD>(qk, yr + qd + (size_t)it.kvh * HD, qk.kn, lane);
-    if (have) *reinterpret_cast<f4*>(kst + 4 * lane) = v;
-  }
-  if (newest && wave == 1) {
-    const f4 v = qkv_head<HD>(qk, yr + qd + kvr + (size_t)it.kvh * HD, nullptr, lane);
-    if (have) {
-      uint16_t* dst = qk.vpages + (size_t)slot * kvr + it.kvh * HD;
+// HF rotate-half: y_i = x_i c - x_{i+h} s, y_{i+h} = x_{i+h} c + x_i s; the
+// partner elements are HD/8 lanes away
+template <int HD>
+__device__ __forceinline__ f4 qkv_rotate(f4 v, f4 c, f4 s, int lane) {
+  const bool second = lane & (HD / 8);
+  f4 r;
 #pragma unroll
-      for (int i = 0; i < 4; i++) dst[4 * lane + i] = f2h_bits(v[i]);
+  for (int i = 0; i < 4; i++) {
+    const float w = __shfl_xor(v[i], HD / 8, 64);
+    r[i] = second ? (v[i] * c[i]) + (w * s[i]) : (v[i] * c[i]) - (w * s[i]);
+  }
+  return r;
+}
+
+// The item's q heads, rotated at the row's position, into qst[G][HD], and for
+// the item holding the lane's newest token its K (norm, RoPE) and V as fp16
+// into kvst[2][HD] and to the pages at the slot.  Head tasks 0..G-1 (q), G (K)
+// and G+1 (V) go round robin over the waves.  load() issues every load of a
+// wave (the caller issues its K/V stream behind them), finish() uses them; the
+// caller's barrier publishes the LDS rows.
+template <int HD, int G>
+struct QkvHeads {
+  static constexpr int HALF = HD / 2, NT = (G + 5) / 4;
+  f4 x[NT][4], gain[NT], c, s;  // slices by task
+  __device__ __forceinline__ bool task(int k, int wave, bool newest) const {
+    const int t = wave + 4 * k;
+    return t < G || (t <= G + 1 && newest);
+  }
+  __device__ __forceinline__ void load(const AttnQkv& qk, const AttnItem& it, int n_kv, int lane, int wave, int pos,
+                                       bool newest) {
+    const int kvr = n_kv * HD, qd = n_kv * G * HD;
+    const size_t yr = (size_t)it.b * (qd + 2 * kvr);
+    const int cc = lane < HD / 4 ? lane : 0;
+#pragma unroll
+    for (int k = 0; k < NT; k++) {
+      const int t = wave + 4 * k;
+      if (!task(k, wave, newest)) continue;
+      const size_t src = t < G ? (size_t)(it.kvh * G + t) * HD : (size_t)qd + (t == G ? 0 : kvr) + (size_t)it.kvh * HD;
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        if (i < qk.y.n) x[k][i] = *reinterpret_cast<const f4*>(qk.y.p + i * qk.y.stride + yr + src + 4 * cc);
+      const float* gn = t < G ? qk.qn : qk.kn;
+      if (t <= G && gn) gain[k] = *reinterpret_cast<const f4*>(gn + 4 * cc);
+    }
+    c = *reinterpret_cast<const f4*>(qk.cos_t + (size_t)pos * HALF + (4 * cc) % HALF);
+    s = *reinterpret_cast<const f4*>(qk.sin_t + (size_t)pos * HALF + (4 * cc) % HALF);
+  }
+  __device__ __forceinline__ void finish(const AttnQkv& qk, const AttnItem& it, int n_kv, int lane, int wave, int slot,
+                                         bool newest, float* qst, _Float16* kvst) const {
+    const int kvr = n_kv * HD;
+#pragma unroll
+    for (int k = 0; k < NT; k++) {
+      const int t = wave + 4 * k;
+      if (!task(k, wave, newest)) continue;
+      f4 v;
+      if (qk.y.n == 1) v = x[k][0];
+      else if (qk.y.n == 2) v = sl_comb<2>({x[k][0], x[k][1]});
+      else v = sl_comb<4>(x[k]);
+      if (t <= G) {
+        if (t < G ? qk.qn != nullptr : qk.kn != nullptr) v = qkv_norm<HD>(qk, v, gain[k], lane);
+        v = qkv_rotate<HD>(v, c, s, lane);
+      }
+      if (lane >= HD / 4) continue;
+      if (t < G) {
+        *reinterpret_cast<f4*>(qst + t * HD + 4 * lane) = v;
+      } else {
+        const h4 hv = {(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+        *reinterpret_cast<h4*>(kvst + (t - G) * HD + 4 * lane) = hv;
+        uint16_t* dst = (t == G ? qk.kpages : qk.vpages) + (size_t)slot * kvr + it.kvh * HD;
+        *reinterpret_cast<h4*>(dst + 4 * lane) = hv;
+      }
     }
   }
-  __syncthreads();
-  // HF rotate-half: y_i = x_i c - x_{i+h} s, y_{i+h} = x_{i+h} c + x_i s
-  const float* ct = qk.cos_t + (size_t)pos * HALF;
-  const float* stt = qk.sin_t + (size_t)pos * HALF;
-  for (int h = wave; h < G; h += 4)
-    for (int i = lane; i < HALF; i += 64) {
-      const float a = qst[h * HD + i], b = qst[h * HD + i + HALF], c = ct[i], sn = stt[i];
-      qst[h * HD + i] = (a * c) - (b * sn);
-      qst[h * HD + i + HALF] = (b * c) + (a * sn);
+};
+
+// Sums of G heads over the 16 lanes of a token (lane j holds slice jp(j)): the
+// slice tree's levels 8, 4, 2, 1 as DPP adds.  While a lane carries more than
+// one head, each level also halves them: lanes with the level's bit clear keep
+// the lower heads and take their partner's values of those, so the four levels
+// cost 11 instructions for four heads instead of 16.  Returns the sum of head
+// qk_head(j).
+template <int G>
+__device__ __forceinline__ int qk_head(int j) {
+  return G == 8 ? j >> 1 : G == 4 ? j >> 2 : G == 2 ? j >> 3 : 0;
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp_f(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+template <int CTRL, int BIT, int N>
+__device__ __forceinline__ void qk_level(float (&v)[N], int n, int j) {
+  if (n >= 2) {
+#pragma unroll
+    for (int h = 0; h < N / 2; h++) {
+      if (2 * h < n) {
+        const float lo = v[h], hi = v[h + n / 2];
+        const float keep = j & BIT ? hi : lo, send = j & BIT ? lo : hi;
+        v[h] = keep + dpp_f<CTRL>(send);
+      }
     }
-  if (newest && wave == 0) {
-    uint16_t* dst = qk.kpages + (size_t)slot * kvr + it.kvh * HD;
-    for (int i = lane; i < HALF; i += 64) {
-      const float a = kst[i], b = kst[i + HALF], c = ct[i], sn = stt[i];
-      dst[i] = f2h_bits((a * c) - (b * sn));
-      dst[i + HALF] = f2h_bits((b * c) + (a * sn));
-    }
+  } else {
+    v[0] = v[0] + dpp_f<CTRL>(v[0]);
   }
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the K/V stores are complete
-  __syncthreads();                     // rotated q in LDS; the appended row is visible to the DMAs that follow
+}
+template <int G>
+__device__ __forceinline__ float qk_tree(float (&v)[G], int j) {
+  qk_level<0x128, 8>(v, G, j);                            // row_ror:8, lanes j and j ^ 8
+  qk_level<0x141, 4>(v, G / 2 > 0 ? G / 2 : 1, j);        // half-row mirror, slices jp and jp ^ 4
+  qk_level<0x4E, 2>(v, G / 4 > 0 ? G / 4 : 1, j);         // quad permutes
+  qk_level<0xB1, 1>(v, 1, j);
+  return v[0];
 }
 
 // ---- few-item attention: one workgroup of four waves per item -------------------
 // The same canonical order as k_attn_split, for launches whose whole work list
-// fits in two rounds of resident workgroups (few lanes, short contexts).  There
-// an item's own instruction stream bounds the launch: a single wave spends
-// ~0.85 us of dependent QK/PV work per 16-token chunk.  Here four waves share
-// each item:
-//  - QK: 16 lanes per token (lane j holds pieces j + 16i, i.e. slice j, in
-//    order), so each wave scores 4 tokens of a chunk; the slice tree runs on
-//    bits 3, 2, 1, 0 as in the one-wave kernel;
-//  - the split's max is exchanged through LDS, and all 256 threads run the
-//    exp pass;
-//  - PV: wave g carries lane group g's chains (tokens t = g mod 4 in order)
-//    with 64 lanes of HD/64 dims each; the groups combine as ((0+1)+(2+3))
-//    through LDS, the same sums as the one-wave kernel's lane exchanges.
-// A ring of RB chunks, each filled by all 256 threads' DMAs, streams the
-// item's K then V chunks and drains between items.  Every list position is
-// static (attn_static_rounds gives one or two rounds here), so no claims.
+// fits in a few rounds of resident workgroups (few lanes, short contexts).
+// There an item's own latency bounds the launch, so a segment of NC 16-token
+// chunks of both K and V is loaded straight into registers at once, before the
+// query is even formed, and the four waves meet at four barriers per item:
+//  - QK: wave w scores tokens 4w..4w+3 of every chunk, 16 lanes per token (lane
+//    j holds the 16-byte pieces of slice jp(j)); the slice tree is DPP adds;
+//  - the split's max is exchanged through LDS, and all 256 threads run the exp
+//    pass;
+//  - PV: wave g carries token group t mod 4 = g in order, HD/64 dims per lane;
+//    the groups combine as ((0+1)+(2+3)) through LDS, the same sums as the
+//    one-wave kernel's lane exchanges.
+// Bound by the chain of dependent loads in front (list entry, page ids and
+// query, rows: ~3 us) and the rows' own streaming.  Measured on MI355X, us a
+// launch, against a ring of 16-token chunks shared by the waves with a barrier
+// per chunk: five Qwen3-0.6B lanes (11.6 k tokens, 47 MB) 15.5 vs 22.7, seven
+// Llama-3-8B lanes 18 vs 28.9, one lane at split 64 7.5 vs 11.1, one
+// Gemma-3-270M lane of 64 tokens 10 vs 13.5.  On long lists the one-wave
+// kernel streams better (128 Llama-3-8B lanes 217 vs 274 us, 45 lanes 87 vs
+// 99), because a workgroup here has nothing in flight while it computes.
+// Every list position is static here, so no claims.
 //
 // QKV: the item's query comes from the qkv projection slices through
-// attn_qkv_prologue (q is unused), and the lane's newest K/V row is appended
-// by the item that holds it, so no separate qkv launch precedes this one.
-// (The QKV form keeps three waves per SIMD for G <= 4: a few kernel-constant
-// prologue values then live in scratch and are reloaded once per item.)
-template <int HD, int G, int RB, bool QKV = false, bool DIRECT = false>
-__global__ __launch_bounds__(256, QKV && G <= 4 ? 3 : 1) void k_attn_split_wg(
+// attn_qkv_prologue (q is unused); the lane's newest K/V row is appended by the
+// item that holds it, which takes the row from LDS, not from the page.
+template <int HD, int G, int NC, bool QKV = false, bool DIRECT = false>
+__global__ __launch_bounds__(256, QKV ? (NC == 4 && G <= 4 && HD == 128 ? 3 : 1)
+                                      : (NC == 4 && G <= 4 && HD == 128 ? 4 : 2)) void k_attn_item(
     int n_kv, int page_size, int ps_shift, int pps, float scale,
     const float* __restrict__ q, const uint16_t* kp, const uint16_t* vp,
     const int32_t* __restrict__ page_table, const int32_t* __restrict__ n_items,
     const int4* __restrict__ items, float* __restrict__ part, AttnQkv qk, AttnOut ao) {
-  constexpr int NP = HD / 8;       // 16-byte pieces per row
-  constexpr int CT = 16;           // tokens per chunk
-  constexpr int CU16 = CT * NP;    // 16-byte units per chunk
-  constexpr int UPT = CU16 / 256;  // DMA units per thread per chunk
-  constexpr int NCL = NP / 16;     // QK pieces per lane
+  constexpr int NCL = HD / 128;    // QK pieces per lane
   constexpr int DPL = HD / 64;     // PV dims per lane
   constexpr int PF = attn_part_floats(HD);
-  static_assert(UPT >= 1 && NCL >= 1 && DPL >= 2, "head dim 128 or 256");
-  static_assert(RB * CU16 * 16 >= 4 * G * HD * 4, "the group combine fits in the ring");
+  typedef _Float16 hv __attribute__((ext_vector_type(DPL)));
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  u32x4* ring = reinterpret_cast<u32x4*>(smem);                   // [RB][CU16]
-  float* red = reinterpret_cast<float*>(ring + RB * CU16);        // [4][G] wave maxima, then l
-  float* qst = red + 4 * G;                                       // [G + 1][HD] q (and K) staging
-  float* sc = qst + (G + 1) * HD;                                 // [split][G] scores
-  float* comb = reinterpret_cast<float*>(smem);                   // [4][G][HD] o, after PV
+  float* comb = reinterpret_cast<float*>(smem);                   // [4][G][HD] o
+  float* qst = comb + 4 * G * HD;                                 // [G][HD] q (QKV)
+  _Float16* kvst = reinterpret_cast<_Float16*>(qst + G * HD);     // [2][HD] the newest K and V row
+  float* red = reinterpret_cast<float*>(kvst + 2 * HD);           // [4][G] wave maxima, then l
+  float* sc = red + 4 * G;                                        // [split][G] scores
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int tt = tid >> 4, j = tid & 15;  // QK: token of the chunk, slice
+  const int g = lane >> 4, j = lane & 15;
+  const int jp = (j & 8) | ((j & 7) < 4 ? (j & 7) : 11 - (j & 7));  // slice: jp ^ 4 sits in the mirrored lane
   const int kvr = n_kv * HD;
   const uint32_t row_bytes = (uint32_t)kvr * 2u;
   const uint32_t page_bytes = (uint32_t)page_size * row_bytes;
+  const uint32_t koff = (uint32_t)(4 * wave + g) * row_bytes + (uint32_t)jp * 16u;
+  const uint32_t voff = (uint32_t)wave * row_bytes + (uint32_t)(lane * DPL * 2);
   const int n_tot = uni(*n_items);
   const int R = gridDim.x, w = blockIdx.x;
-  const int ks = attn_static_rounds(n_tot, R);
-  for (int k = 0; k < ks; k++) {
+  const int rounds = (n_tot + R - 1) / R;
+  for (int k = 0; k < rounds; k++) {
     const int pos = k * R + ((k & 1) ? R - 1 - w : w);
     if (pos >= n_tot) continue;
     const AttnItem it = attn_item_make(items[pos]);
-    const int npos = 2 * it.nch;
-    // The pages of the item's chunks: every wave loads them once per item
-    // (lane i holds page pg0 + i + 64 k in pgv[k]) and reads each chunk's
-    // page with v_readlane (a lookup per chunk would put a memory latency
-    // before every DMA).
+    // The pages of the item's chunks (lane i holds page pg0 + i + 64 k in pgv[k])
     const int pg0 = it.T0 >> ps_shift;
-    const int npg = ((it.T0 + (it.nch - 1) * CT) >> ps_shift) - pg0 + 1;
+    const int npg = ((it.T0 + (it.nch - 1) * 16) >> ps_shift) - pg0 + 1;
     const int32_t* prow = page_table + (size_t)it.b * pps + pg0;
     constexpr int PGV = (RSTR_NCH + 63) / 64;
     int32_t pgv[PGV];
 #pragma unroll
-    for (int k = 0; k < PGV; k++) pgv[k] = (k == 0 || 64 * k < npg) && lane + 64 * k < npg ? prow[lane + 64 * k] : 0;
-    auto issue = [&](int p) {
-      const bool isk = p < it.nch;
-      const int c = isk ? p : p - it.nch;
-      const int tb = it.T0 + c * CT;
-      const int pi = (tb >> ps_shift) - pg0;
+    for (int i = 0; i < PGV; i++) pgv[i] = (i == 0 || 64 * i < npg) && lane + 64 * i < npg ? prow[lane + 64 * i] : 0;
+    int slot = -1, qpos = 0;
+    bool newest = false;
+    if constexpr (QKV) {
+      slot = uni(qk.slots[it.b]);
+      qpos = uni(qk.positions[it.b]);
+      newest = slot >= 0 && it.t1 == uni(qk.lengths[it.b]);
+    }
+    auto chunk_base = [&](const uint16_t* slab, int c) -> const char* {
+      const int tb = it.T0 + c * 16, pi = (tb >> ps_shift) - pg0;
       int page = __builtin_amdgcn_readlane(pgv[0], pi & 63);
 #pragma unroll
-      for (int k = 1; k < PGV; k++)
-        if ((pi >> 6) == k) page = __builtin_amdgcn_readlane(pgv[k], pi & 63);
-      const char* base = reinterpret_cast<const char*>((isk ? kp : vp) + it.kvh * HD) +
-                         (uint64_t)(uint32_t)page * page_bytes + (uint32_t)(tb & (page_size - 1)) * row_bytes;
-      u32x4* dst = ring + (p % RB) * CU16;
+      for (int i = 1; i < PGV; i++)
+        if ((pi >> 6) == i) page = __builtin_amdgcn_readlane(pgv[i], pi & 63);
+      return reinterpret_cast<const char*>(slab + it.kvh * HD) + (uint64_t)(uint32_t)page * page_bytes +
+             (uint32_t)(tb & (page_size - 1)) * row_bytes;
+    };
+    // a segment's rows; chunks past the item re-read its last one
+    u32x4 kr[NC][NCL];
+    hv vr[NC][4];
+    auto load_k = [&](int s0) {
 #pragma unroll
-      for (int u = 0; u < UPT; u++) {
-        const int un = u * 256 + tid;
-        __builtin_amdgcn_global_load_lds(
-            reinterpret_cast<const void*>(base + (uint32_t)(un / NP) * row_bytes + (uint32_t)(un % NP) * 16u),
-            RSTR_LDS_PTR(dst + u * 256 + wave * 64), 16, 0, RSTR_KV_POLICY);
+      for (int c = 0; c < NC; c++) {
+        const char* base = chunk_base(kp, min(s0 + c, it.nch - 1));
+#pragma unroll
+        for (int i = 0; i < NCL; i++) kr[c][i] = ld_stream(reinterpret_cast<const u32x4*>(base + koff + 256 * i));
       }
     };
-    // this thread's query pieces: slice j of each head
+    auto load_v = [&](int s0) {
+#pragma unroll
+      for (int c = 0; c < NC; c++) {
+        const char* base = chunk_base(vp, min(s0 + c, it.nch - 1));
+#pragma unroll
+        for (int rd = 0; rd < 4; rd++)
+          vr[c][rd] = ld_stream(reinterpret_cast<const hv*>(base + voff + (uint32_t)(4 * rd) * row_bytes));
+      }
+    };
+    // Query loads first, then the K/V stream: loads return in issue order, so
+    // QK runs while V is still arriving.
     float qv[G][NCL][8];
+    auto read_q = [&](const float* qg) {
+#pragma unroll
+      for (int h = 0; h < G; h++)
+#pragma unroll
+        for (int i = 0; i < NCL; i++) {
+          const f4 a = *reinterpret_cast<const f4*>(qg + h * HD + 8 * (jp + 16 * i));
+          const f4 b4 = *reinterpret_cast<const f4*>(qg + h * HD + 8 * (jp + 16 * i) + 4);
+#pragma unroll
+          for (int e = 0; e < 4; e++) { qv[h][i][e] = a[e]; qv[h][i][4 + e] = b4[e]; }
+        }
+    };
     if constexpr (QKV) {
-      attn_qkv_prologue<HD, G>(qk, it, n_kv, lane, wave, qst);
-#pragma unroll
-      for (int h = 0; h < G; h++)
-#pragma unroll
-        for (int i = 0; i < NCL; i++) {
-          const f4 a = *reinterpret_cast<const f4*>(qst + h * HD + 8 * (j + 16 * i));
-          const f4 b4 = *reinterpret_cast<const f4*>(qst + h * HD + 8 * (j + 16 * i) + 4);
-#pragma unroll
-          for (int e = 0; e < 4; e++) { qv[h][i][e] = a[e]; qv[h][i][4 + e] = b4[e]; }
-        }
+      QkvHeads<HD, G> heads;
+      heads.load(qk, it, n_kv, lane, wave, qpos, newest);
+      __asm__ __volatile__("" ::: "memory");
+      load_k(0);
+      load_v(0);
+      __asm__ __volatile__("" ::: "memory");
+      heads.finish(qk, it, n_kv, lane, wave, slot, newest, qst, kvst);
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0); the loads in flight stay so
+      __asm__ __volatile__("" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      __asm__ __volatile__("" ::: "memory");
+      read_q(qst);
     } else {
-      const float* qg = q + ((size_t)it.b * (n_kv * G) + it.kvh * G) * HD;
-#pragma unroll
-      for (int h = 0; h < G; h++)
-#pragma unroll
-        for (int i = 0; i < NCL; i++) {
-          const f4 a = *reinterpret_cast<const f4*>(qg + h * HD + 8 * (j + 16 * i));
-          const f4 b4 = *reinterpret_cast<const f4*>(qg + h * HD + 8 * (j + 16 * i) + 4);
-#pragma unroll
-          for (int e = 0; e < 4; e++) { qv[h][i][e] = a[e]; qv[h][i][4 + e] = b4[e]; }
-        }
+      read_q(q + ((size_t)it.b * (n_kv * G) + it.kvh * G) * HD);
+      __asm__ __volatile__("" ::: "memory");
+      load_k(0);
+      load_v(0);
+      __asm__ __volatile__("" ::: "memory");
     }
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // page ids and the query pieces have arrived
-    for (int p = 0; p < RB - 1 && p < npos; p++) issue(p);
-    float mx[G], o[G][DPL], l[G];
+    const int tn = it.t1 - 1, cn = newest ? (tn - it.T0) >> 4 : -1;  // the newest token and its chunk
+    // ---- QK ---------------------------------------------------------------------
+    float mx = -__builtin_inff();
+    for (int s0 = 0; s0 < it.nch; s0 += NC) {
+      if (s0 > 0) load_k(s0);
 #pragma unroll
-    for (int h = 0; h < G; h++) {
-      mx[h] = -__builtin_inff();
-      l[h] = 0.0f;
+      for (int c0 = 0; c0 < NC; c0 += 2) {
+        if (s0 + c0 >= it.nch) break;  // chunks in pairs; one past the item scores nothing
+#pragma unroll
+        for (int c = c0; c < c0 + 2; c++) {
+          const int t = it.T0 + (s0 + c) * 16 + 4 * wave + g;
+          if constexpr (QKV) {
+            if (s0 + c == cn && t == tn) {
+#pragma unroll
+              for (int i = 0; i < NCL; i++) kr[c][i] = *reinterpret_cast<const u32x4*>(kvst + 8 * (jp + 16 * i));
+            }
+          }
+          float sv[G];
+#pragma unroll
+          for (int h = 0; h < G; h++) sv[h] = 0.0f;
+#pragma unroll
+          for (int i = 0; i < NCL; i++) {
+            const h8 kv = __builtin_bit_cast(h8, kr[c][i]);
+#pragma unroll
+            for (int h = 0; h < G; h++)
+#pragma unroll
+              for (int e = 0; e < 8; e++) sv[h] = __builtin_fmaf(qv[h][i][e], (float)kv[e], sv[h]);
+          }
+          const float s = qk_tree<G>(sv, j) * scale;
+          const bool valid = t >= it.t0 && t < it.t1;
+          mx = fmaxf(mx, valid ? s : -__builtin_inff());
+          if (valid && j % (16 / G) == 0) sc[(t - it.t0) * G + qk_head<G>(j)] = s;
+        }
+      }
+    }
+    // ---- softmax numerators over the split ------------------------------------------
+    mx = xor_max<32>(xor_max<16>(mx));
+    if (g == 0 && j % (16 / G) == 0) red[wave * G + qk_head<G>(j)] = mx;
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __asm__ __volatile__("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    __asm__ __volatile__("" ::: "memory");
+    const int nt = it.t1 - it.t0, eh = tid % G;
+    const float m = fmaxf(fmaxf(red[eh], red[G + eh]), fmaxf(red[2 * G + eh], red[3 * G + eh]));  // of head eh
+    for (int i = tid; i < nt * G; i += 256) sc[i] = dexp(sc[i] - m);
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __asm__ __volatile__("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    __asm__ __volatile__("" ::: "memory");
+    // ---- PV: wave g = lane group g, rows 4 rd + g of each chunk ------------------------
+    float o[G][DPL], l = 0.0f;  // l of head eh
+#pragma unroll
+    for (int h = 0; h < G; h++)
 #pragma unroll
       for (int d = 0; d < DPL; d++) o[h][d] = 0.0f;
-    }
-    for (int p = 0; p < npos; p++) {
-      // chunk p has landed for this thread once at most the DMAs of the
-      // positions after it (at most RB - 2) are outstanding; its LDS writes
-      // (scores, exp values) are done before the barrier
-      if (p + RB - 2 < npos) __builtin_amdgcn_s_waitcnt(((UPT * (RB - 2)) & 0xF) | (((UPT * (RB - 2)) >> 4) << 14) | 0x0070);
-      else __builtin_amdgcn_s_waitcnt(0x0070);
-      __asm__ __volatile__("" ::: "memory");
-      __builtin_amdgcn_s_barrier();  // every thread's part of chunk p, and every read of slot (p-1) % RB, is done
-      __asm__ __volatile__("" ::: "memory");
-      if (p + RB - 1 < npos) issue(p + RB - 1);
-      const u32x4* buf = ring + (p % RB) * CU16;
-      if (p < it.nch) {
-        // ---- QK: token tt of chunk p, slice j -----------------------------------
-        const int t = it.T0 + p * CT + tt;
-        const bool valid = t >= it.t0 && t < it.t1;
-        float sv[G];
+    for (int s0 = 0; s0 < it.nch; s0 += NC) {
+      if (s0 > 0) load_v(s0);
 #pragma unroll
-        for (int h = 0; h < G; h++) sv[h] = 0.0f;
+      for (int c = 0; c < NC; c++) {
+        if (s0 + c >= it.nch) break;
+        const int tb = it.T0 + (s0 + c) * 16 + wave;
+        hv v[4];
+        float p[4][G], pl[4];
 #pragma unroll
-        for (int i = 0; i < NCL; i++) {
-          const h8 kv = __builtin_bit_cast(h8, buf[tt * NP + j + 16 * i]);
+        for (int rd = 0; rd < 4; rd++) v[rd] = vr[c][rd];
+        auto read_p = [&](int rd, int at) {
+          const float* ps = sc + at * G;
+          if constexpr (G % 4 == 0) {
+#pragma unroll
+            for (int h4 = 0; h4 < G; h4 += 4) {
+              const f4 p4 = *reinterpret_cast<const f4*>(ps + h4);
+#pragma unroll
+              for (int e = 0; e < 4; e++) p[rd][h4 + e] = p4[e];
+            }
+          } else {
+#pragma unroll
+            for (int h = 0; h < G; h++) p[rd][h] = ps[h];
+          }
+          pl[rd] = ps[eh];
+        };
+        if (tb - wave >= it.t0 && tb - wave + 16 <= it.t1 && s0 + c != cn) {
+#pragma unroll
+          for (int rd = 0; rd < 4; rd++) read_p(rd, tb + 4 * rd - it.t0);
+        } else {
+          // a row outside [t0, t1) contributes p = 0 times v = 0, which leaves
+          // o and l unchanged (they are never -0)
+#pragma unroll
+          for (int rd = 0; rd < 4; rd++) {
+            const int t = tb + 4 * rd;
+            const bool ok = t >= it.t0 && t < it.t1;
+            read_p(rd, ok ? t - it.t0 : 0);
+            if constexpr (QKV) {
+              if (newest && t == tn) v[rd] = *reinterpret_cast<const hv*>(kvst + HD + lane * DPL);
+            }
+#pragma unroll
+            for (int h = 0; h < G; h++) p[rd][h] = ok ? p[rd][h] : 0.0f;
+            pl[rd] = ok ? pl[rd] : 0.0f;
+#pragma unroll
+            for (int d = 0; d < DPL; d++) v[rd][d] = ok ? v[rd][d] : (_Float16)0.0f;
+          }
+        }
+#pragma unroll
+        for (int rd = 0; rd < 4; rd++) {
+          l = l + pl[rd];
 #pragma unroll
           for (int h = 0; h < G; h++)
 #pragma unroll
-            for (int e = 0; e < 8; e++) sv[h] = __builtin_fmaf(qv[h][i][e], (float)kv[e], sv[h]);
-        }
-#pragma unroll
-        for (int h = 0; h < G; h++) {
-          // slice tree inside each 16-lane row, all DPP: row_ror:8 is lane
-          // i ^ 8; after that level lanes i and i ^ 8 agree, so row_ror:4
-          // delivers the value of lane i ^ 4
-          float v = sv[h];
-          v = v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xF, 0xF, true));
-          v = v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x124, 0xF, 0xF, true));
-          v = v + xor_lane<2>(v);
-          v = v + xor_lane<1>(v);
-          const float s = v * scale;
-          if (valid) mx[h] = fmaxf(mx[h], s);
-          if (valid && j == 0) sc[(size_t)(t - it.t0) * G + h] = s;
-        }
-        if (p == it.nch - 1) {
-          // ---- softmax numerators over the split --------------------------------
-#pragma unroll
-          for (int h = 0; h < G; h++) {
-            mx[h] = wave_max(mx[h]);
-            if (lane == 0) red[wave * G + h] = mx[h];
-          }
-          // scores and wave maxima are written (LDS only: the V chunks in
-          // flight keep streaming)
-          __builtin_amdgcn_s_waitcnt(0xC07F);
-          __asm__ __volatile__("" ::: "memory");
-          __builtin_amdgcn_s_barrier();
-          __asm__ __volatile__("" ::: "memory");
-#pragma unroll
-          for (int h = 0; h < G; h++) mx[h] = fmaxf(fmaxf(red[h], red[G + h]), fmaxf(red[2 * G + h], red[3 * G + h]));
-          const int nt = it.t1 - it.t0;
-          for (int i = tid; i < nt; i += 256)
-#pragma unroll
-            for (int h = 0; h < G; h++) sc[i * G + h] = dexp(sc[i * G + h] - mx[h]);
-          // the next iteration's barrier orders these writes before PV reads them
-        }
-      } else {
-        // ---- PV: wave g = lane group g, rows r = 4 rd + g of the chunk -------------
-        const int c = p - it.nch;
-        const unsigned char* vb = reinterpret_cast<const unsigned char*>(buf);
-#pragma unroll
-        for (int rd = 0; rd < CT / 4; rd++) {
-          const int r = rd * 4 + wave;
-          const int t = it.T0 + c * CT + r;
-          const bool ok = t >= it.t0 && t < it.t1;
-          float vv[DPL];
-          if constexpr (DPL == 2) {
-            const h2 hv = *reinterpret_cast<const h2*>(vb + r * HD * 2 + lane * DPL * 2);
-            vv[0] = ok ? (float)hv[0] : 0.0f;
-            vv[1] = ok ? (float)hv[1] : 0.0f;
-          } else {
-            const h4 hv = *reinterpret_cast<const h4*>(vb + r * HD * 2 + lane * DPL * 2);
-#pragma unroll
-            for (int e = 0; e < 4; e++) vv[e] = ok ? (float)hv[e] : 0.0f;
-          }
-          const float* ps = sc + (size_t)(ok ? t - it.t0 : 0) * G;
-#pragma unroll
-          for (int h = 0; h < G; h++) {
-            const float pr = ok ? ps[h] : 0.0f;
-            l[h] = l[h] + pr;
-#pragma unroll
-            for (int d = 0; d < DPL; d++) o[h][d] = __builtin_fmaf(pr, vv[d], o[h][d]);
-          }
+            for (int d = 0; d < DPL; d++) o[h][d] = __builtin_fmaf(p[rd][h], (float)v[rd][d], o[h][d]);
         }
       }
     }
     // ---- combine the four groups ((0+1)+(2+3)) and write the partial ------------
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();  // every read of the ring is done: it becomes the combine buffer
 #pragma unroll
-    for (int h = 0; h < G; h++) {
+    for (int h = 0; h < G; h++)
 #pragma unroll
       for (int d = 0; d < DPL; d++) comb[(wave * G + h) * HD + lane * DPL + d] = o[h][d];
-      if (lane == 0) red[wave * G + h] = l[h];
-    }
+    // every wave has read red before the exp pass's barrier: it takes l now
+    if (lane < G) red[wave * G + lane] = l;
     __syncthreads();
+    // maxima per head again, from the thread that holds them
     if constexpr (DIRECT) {
       // The lane's whole visible range is this one split: k_attn_merge's sums
       // for one partial (w = exp(m - M) with M = m, L = fmaf(l, w, 0),
@@ -2776,20 +2857,17 @@ __global__ __launch_bounds__(256, QKV && G <= 4 ? 3 : 1) void k_attn_split_wg(
       const int nb = n_kv * G * HD / 32;
       for (int e = tid; e < G * HD / 8; e += 256) {
         const int h = e / (HD / 8), d8 = (e % (HD / 8)) * 8;
-        float m = mx[0];
-#pragma unroll
-        for (int k = 1; k < G; k++)
-          if (h == k) m = mx[k];
         const float* lc = red;
-        const float w = dexp(m - m);
-        const float L = __builtin_fmaf((lc[h] + lc[G + h]) + (lc[2 * G + h] + lc[3 * G + h]), w, 0.0f);
+        const float mh = __shfl(m, h, 64);  // lane h of every wave holds head h (G <= 8)
+        const float wgt = dexp(mh - mh);
+        const float L = __builtin_fmaf((lc[h] + lc[G + h]) + (lc[2 * G + h] + lc[3 * G + h]), wgt, 0.0f);
         float O[8];
         float a = 0.0f;
 #pragma unroll
         for (int i = 0; i < 8; i++) {
           const int c = h * HD + d8 + i;
-          const float o = (comb[0 * G * HD + c] + comb[1 * G * HD + c]) + (comb[2 * G * HD + c] + comb[3 * G * HD + c]);
-          O[i] = __builtin_fmaf(o, w, 0.0f) / L;
+          const float ov = (comb[0 * G * HD + c] + comb[1 * G * HD + c]) + (comb[2 * G * HD + c] + comb[3 * G * HD + c]);
+          O[i] = __builtin_fmaf(ov, wgt, 0.0f) / L;
           a = fmaxf(a, fabsf(O[i]));
         }
         a = fmaxf(a, xor_lane<1>(a));
@@ -2799,39 +2877,34 @@ __global__ __launch_bounds__(256, QKV && G <= 4 ? 3 : 1) void k_attn_split_wg(
         const int b = it.b;
         const int kcol0 = (it.kvh * G + h) * HD + d8;
         const int blk = kcol0 >> 5, g8 = (kcol0 & 31) >> 3;
-        h8 qv;
+        h8 qo;
 #pragma unroll
         for (int i = 0; i < 8; i++) {
           float v = __builtin_rintf(O[i] * id);
           v = fminf(127.0f, fmaxf(-127.0f, v));
-          qv[i] = (_Float16)(v * dq);
+          qo[i] = (_Float16)(v * dq);
         }
-        *reinterpret_cast<h8*>(ao.q + ((((size_t)(b >> 4) * nb + blk) * 4 + g8) * 16 + (b & 15)) * 8) = qv;
+        *reinterpret_cast<h8*>(ao.q + ((((size_t)(b >> 4) * nb + blk) * 4 + g8) * 16 + (b & 15)) * 8) = qo;
         if (g8 == 0) ao.s[(size_t)blk * ao.mpad + b] = dq;
       }
-      __syncthreads();  // the combine buffer is read before the next item's DMA refills the ring
-      continue;
-    }
-    float* rec = part + (size_t)it.idx * G * PF;
-    for (int e = tid; e < G * HD / 4; e += 256) {
-      const int h = e / (HD / 4), d4 = (e % (HD / 4)) * 4;
-      f4 out;
+    } else {
+      float* rec = part + (size_t)it.idx * G * PF;
+      for (int e = tid; e < G * HD / 4; e += 256) {
+        const int h = e / (HD / 4), d4 = (e % (HD / 4)) * 4;
+        f4 out;
 #pragma unroll
-      for (int i = 0; i < 4; i++)
-        out[i] = (comb[(0 * G + h) * HD + d4 + i] + comb[(1 * G + h) * HD + d4 + i]) +
-                 (comb[(2 * G + h) * HD + d4 + i] + comb[(3 * G + h) * HD + d4 + i]);
-      *reinterpret_cast<f4*>(rec + h * PF + d4) = out;
+        for (int i = 0; i < 4; i++)
+          out[i] = (comb[(0 * G + h) * HD + d4 + i] + comb[(1 * G + h) * HD + d4 + i]) +
+                   (comb[(2 * G + h) * HD + d4 + i] + comb[(3 * G + h) * HD + d4 + i]);
+        *reinterpret_cast<f4*>(rec + h * PF + d4) = out;
+      }
+      if (tid < G) {
+        const float* lc = red;
+        rec[tid * PF + HD] = m;
+        rec[tid * PF + HD + 1] = (lc[tid] + lc[G + tid]) + (lc[2 * G + tid] + lc[3 * G + tid]);
+      }
     }
-    if (tid < G) {
-      const float* lc = red;
-      float m = mx[0];
-#pragma unroll
-      for (int h = 1; h < G; h++)
-        if (tid == h) m = mx[h];
-      rec[tid * PF + HD] = m;
-      rec[tid * PF + HD + 1] = (lc[tid] + lc[G + tid]) + (lc[2 * G + tid] + lc[3 * G + tid]);
-    }
-    __syncthreads();  // the combine buffer is read before the next item's DMA refills the ring
+    __syncthreads();  // comb, red and qst are read before the next item writes them
   }
 }
 
@@ -3196,13 +3269,18 @@ struct AttnSplit {
     return n;
   }
   static int ring(const AttnGeom& g) { return waves_per_cu(g, RBS) > waves_per_cu(g, RB) ? RBS : RB; }
-  // Few-item launches (k_attn_split_wg, one 4-wave workgroup per item): head
-  // dim 128 or 256, whole-page chunks, and a largest work list that fits in
-  // two rounds of resident workgroups.  Its ring is 32 KB deep.
+  // Few-item launches (k_attn_item, one 4-wave workgroup per item): head dim
+  // 128 or 256, whole-page chunks, and a largest work list that fits in two
+  // rounds of resident workgroups.  Its segments hold 64 tokens for splits up
+  // to 64, else 256 (head dim 256: 128), as far as a thread's registers go.
   static constexpr bool kWG = HD == 128 || HD == 256;
-  static constexpr int RBW = HD == 128 ? 8 : 4;
+  static constexpr int NCB = G == 8 ? 4 : HD == 128 ? 16 : 8;
+  template <bool QKV, bool DIRECT>
+  static decltype(&k_attn_item<HD, G, 4, QKV, DIRECT>) item_kernel(const AttnGeom& g) {
+    return g.split > 64 ? k_attn_item<HD, G, NCB, QKV, DIRECT> : k_attn_item<HD, G, 4, QKV, DIRECT>;
+  }
   static size_t lds_wg(const AttnGeom& g) {
-    return (size_t)RBW * 16 * (HD / 8) * 16 + sizeof(float) * (G * (4 + (size_t)g.split) + (G + 1) * HD);
+    return sizeof(float) * (size_t)(4 * G * HD + G * HD + HD + 4 * G + G * g.split);
   }
   template <bool QKV = false>
   static int wg_capacity(const AttnGeom& g) {
@@ -3210,8 +3288,7 @@ struct AttnSplit {
       return 0;
     } else {
       int n = 0;
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_attn_split_wg<HD, G, RBW, QKV>, 256, lds_wg(g)) !=
-          hipSuccess)
+      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, item_kernel<QKV, false>(g), 256, lds_wg(g)) != hipSuccess)
         return 0;
       return device_cus() * n;
     }
@@ -3243,13 +3320,10 @@ struct AttnSplit {
     const int shift = pg16(g) ? __builtin_ctz((unsigned)g.page_size) : 0;
     if constexpr (kWG) {
       if (use_wg(g, max_items)) {
-        if (out)
-          hipLaunchKernelGGL((k_attn_split_wg<HD, G, RBW, false, true>), dim3(R), dim3(256), lds_wg(g), st, g.n_kv,
-                             g.page_size, shift, g.pps, g.scale, q, kp, vp, pt, n_items, items, part, AttnQkv{},
-                             *out);
-        else
-          hipLaunchKernelGGL((k_attn_split_wg<HD, G, RBW>), dim3(R), dim3(256), lds_wg(g), st, g.n_kv, g.page_size,
-                             shift, g.pps, g.scale, q, kp, vp, pt, n_items, items, part, AttnQkv{}, AttnOut{});
+        const AttnOut ao = out ? *out : AttnOut{};
+        const auto kern = out ? item_kernel<false, true>(g) : item_kernel<false, false>(g);
+        hipLaunchKernelGGL(kern, dim3(R), dim3(256), lds_wg(g), st, g.n_kv, g.page_size, shift, g.pps, g.scale, q, kp,
+                           vp, pt, n_items, items, part, AttnQkv{}, ao);
         return;
       }
     }
@@ -3266,14 +3340,10 @@ struct AttnSplit {
       const int32_t* n_items = tab + 4 * g.batch;
       const int4* items = reinterpret_cast<const int4*>(tab + attn_items_offset(g.batch));
       const int shift = __builtin_ctz((unsigned)g.page_size);
-      if (out)
-        hipLaunchKernelGGL((k_attn_split_wg<HD, G, RBW, true, true>), dim3(R), dim3(256), lds_wg(g), st, g.n_kv,
-                           g.page_size, shift, g.pps, g.scale, nullptr, qk.kpages, qk.vpages, pt, n_items, items,
-                           part, qk, *out);
-      else
-        hipLaunchKernelGGL((k_attn_split_wg<HD, G, RBW, true>), dim3(R), dim3(256), lds_wg(g), st, g.n_kv,
-                           g.page_size, shift, g.pps, g.scale, nullptr, qk.kpages, qk.vpages, pt, n_items, items,
-                           part, qk, AttnOut{});
+      const AttnOut ao = out ? *out : AttnOut{};
+      const auto kern = out ? item_kernel<true, true>(g) : item_kernel<true, false>(g);
+      hipLaunchKernelGGL(kern, dim3(R), dim3(256), lds_wg(g), st, g.n_kv, g.page_size, shift, g.pps, g.scale, nullptr,
+                         qk.kpages, qk.vpages, pt, n_items, items, part, qk, ao);
       return true;
     } else {
       return false;
