@@ -54,6 +54,7 @@ struct Slices {
   size_t stride;
 };
 int qgemm_splits(int n, int mpad, int bits);
+int qgemm_head_splits(int n, int k, int rows, int bits);  // of the LM head: 1, or 4 for launch_argmax_gather to add
 hipError_t launch_qgemm(hipStream_t st, const QTensor& w, const ActBuf& x, int m_rows, float* y,
                         int ldy, int splits, size_t slice_stride);
 // Gate/up (w = [gate | up], n = 2*ff) with act(gate)*up quantised into `out`
@@ -201,7 +202,8 @@ hipError_t launch_attn_merge(hipStream_t st, const AttnGeom& g, const int32_t* l
 // Segments per row of the tail's first stage; the candidate buffer holds
 // rows * argmax_segments(rows, vocab) (value, index) pairs of int32 words.
 int argmax_segments(int rows, int vocab);
-hipError_t launch_argmax_gather(hipStream_t st, const float* logits, int rows, int vocab,
+// Logits in one slice, or in four whose sums are written to `out`.
+hipError_t launch_argmax_gather(hipStream_t st, Slices logits, float* out, int rows, int vocab,
                                 const float* emb, int d, int32_t* tok, float* r0, int32_t* cand);
 hipError_t launch_gather_rows(hipStream_t st, const float* emb, int d, const int32_t* lanes,
                               const int32_t* tokens, int n, float* r0);

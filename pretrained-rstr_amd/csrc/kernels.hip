@@ -1026,6 +1026,120 @@ hipError_t launch_qgemv_wg(hipStream_t st, const QTensor& w, const ActBuf& x, in
   return qgemv_wg_go<false>(st, w, x, m_rows, y, ldy, splits, slice_stride, ActIn{});
 }
 
+// ---- 2..16 rows against a long K: weights streamed past resident activations ------
+// A narrow projection over a long K (the MLP down projection) has one quarter
+// chain per wave and about one wave per SIMD, so k_qgemm's chunk loop paid a
+// memory latency per chunk (one chunk ahead, a barrier each: 28 chunks of ~0.7
+// us).  Here the quarter's activation fragments (qs KB) are brought to LDS once
+// and the chunk loop has no barrier: each wave streams the weights of its 16
+// columns through D chunks of registers, reloading a slot as soon as it is
+// used.  Same fragments, block dots and chain as k_qgemm with NQ = 1.  Measured
+// on MI355X, 4096 x 14336 Q4 at 7 and 16 rows: 19.8 -> 13.4 and 20.0 -> 13.7 us.
+// Launches with several waves per SIMD (gate/up, qkv, o) hide that latency
+// among the waves and were slower in this form (gate/up 16.9 -> 18.6 us, qkv
+// 7.3 -> 8.0), as were 32 and 48 rows (gate/up 22.9 -> 29.3, 34.4 -> 51.8).
+template <int BITS, int D>
+__global__ __launch_bounds__(256, 2) void k_qgemm_res(const uint32_t* __restrict__ W, const uint16_t* __restrict__ Ws,
+                                                      const _Float16* __restrict__ X, int nb, int nct,
+                                                      float* __restrict__ Y, int ldy, int m_rows,
+                                                      size_t slice_stride) {
+  constexpr int DW = BITS == 4 ? 1 : 2;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  u32x4* xa = reinterpret_cast<u32x4*>(smem);  // [qs][64]
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nn = lane & 15, g = lane >> 4;
+  const int ct = blockIdx.x * 4 + wave, split = blockIdx.y;
+  const int nb4 = nb >> 2, qs = nb >> 2, nchunk = qs >> 2;  // nchunk is a multiple of D
+  const int b_begin = split * qs;
+  const uint32_t E = opaque_vgpr(0x64006400u);
+  for (int b = wave; b < qs; b += 4)
+    __builtin_amdgcn_global_load_lds(reinterpret_cast<const void*>(X + (size_t)(b_begin + b) * 512 + lane * 8),
+                                     RSTR_LDS_PTR(xa + b * 64), 16, 0, 0);
+  const int ctl = min(ct, nct - 1);
+  const uint32_t* wsrc = W + ((size_t)ctl * nb4 + (b_begin >> 2)) * 256 * DW + (g * 16 + nn) * 4 * DW;
+  const uint32_t* ssrc = reinterpret_cast<const uint32_t*>(Ws + ((size_t)ctl * nb4 + (b_begin >> 2)) * 64) + g * 8;
+  uint32_t pw[D][4 * DW], ps[D][8];
+  auto load = [&](int d, int ch) {
+    ch = min(ch, nchunk - 1);
+    const uint32_t* wp = wsrc + (size_t)ch * 256 * DW;
+    const uint32_t* sp = ssrc + (size_t)ch * 32;
+    const u32x4 w0 = ld_stream(reinterpret_cast<const u32x4*>(wp));
+#pragma unroll
+    for (int k = 0; k < 4; k++) pw[d][k] = w0[k];
+    if constexpr (DW == 2) {
+      const u32x4 w1 = ld_stream(reinterpret_cast<const u32x4*>(wp + 4));
+#pragma unroll
+      for (int k = 0; k < 4; k++) pw[d][4 + k] = w1[k];
+    }
+    const u32x4 s0 = ld_stream(reinterpret_cast<const u32x4*>(sp));
+    const u32x4 s1 = ld_stream(reinterpret_cast<const u32x4*>(sp + 4));
+#pragma unroll
+    for (int k = 0; k < 4; k++) { ps[d][k] = s0[k]; ps[d][4 + k] = s1[k]; }
+  };
+#pragma unroll
+  for (int d = 0; d < D; d++) load(d, d);
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's fragments (and first chunks)
+  __syncthreads();                     // every wave's fragments
+  float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  const f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int c0 = 0; c0 < nchunk; c0 += D) {
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+      const u32x4* xc = xa + (size_t)(c0 + d) * 256 + lane;
+      f4 t[4];
+#pragma unroll
+      for (int kc = 0; kc < 4; kc++) {
+        h8 wv;
+        if constexpr (BITS == 4) wv = unpack_q4(pw[d][kc], E);
+        else wv = unpack_q8(pw[d][2 * kc], pw[d][2 * kc + 1], E);
+        t[kc] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv, __builtin_bit_cast(h8, xc[kc * 64]), zero, 0, 0, 0);
+      }
+#pragma unroll
+      for (int kc = 0; kc < 4; kc++) {
+        const h2 d0 = __builtin_bit_cast(h2, ps[d][2 * kc]), d1 = __builtin_bit_cast(h2, ps[d][2 * kc + 1]);
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[r] = __builtin_fmaf(t[kc][r], (float)(r < 2 ? d0 : d1)[r & 1], acc[r]);
+      }
+      load(d, c0 + d + D);  // this slot's next chunk (past the end: a re-read of the last)
+    }
+  }
+  if (ct < nct && nn < m_rows)
+    *reinterpret_cast<f4*>(Y + (size_t)split * slice_stride + (size_t)nn * ldy + ct * 16 + 4 * g) =
+        f4{acc[0], acc[1], acc[2], acc[3]};
+}
+
+namespace {
+// The launches k_qgemm_res takes: 2..16 rows, four K slices of at least 14
+// whole chunks (shorter chains are preloaded by k_qgemm), at most one workgroup
+// per CU of a 256-CU device, fragments that fit the LDS.
+bool qgemm_res_serves(const QTensor& w, int mpad, int m_rows, int splits) {
+  const int nb = w.k / 32, nchunk = nb / 16;
+  return mpad == 16 && m_rows >= 2 && splits == 4 && nb % 16 == 0 && nchunk >= 14 && nchunk % 2 == 0 &&
+         (w.n / 16 + 3) / 4 * 4 <= 256 && nb / 4 * 1024 <= 160 * 1024;
+}
+hipError_t launch_qgemm_res(hipStream_t st, const QTensor& w, const ActBuf& x, int m_rows, float* y, int ldy,
+                            size_t slice_stride) {
+  const int nb = w.k / 32, nct = w.n / 16, nchunk = nb / 16;
+  const dim3 grid((nct + 3) / 4, 4);
+  const size_t lds = (size_t)nb / 4 * 1024;
+#define RSTR_RES(B_, D_)                                                                                              \
+  hipLaunchKernelGGL((k_qgemm_res<B_, D_>), grid, dim3(256), lds, st, (const uint32_t*)w.w, w.s, x.q, nb, nct, y, ldy, \
+                     m_rows, slice_stride)
+#define RSTR_RES_D(B_)                            \
+  do {                                            \
+    if (nchunk % 7 == 0) RSTR_RES(B_, 7);         \
+    else if (nchunk % 4 == 0) RSTR_RES(B_, 4);    \
+    else RSTR_RES(B_, 2);                         \
+  } while (0)
+  if (w.bits == 4) RSTR_RES_D(4);
+  else RSTR_RES_D(8);
+#undef RSTR_RES_D
+#undef RSTR_RES
+  return hipGetLastError();
+}
+}  // namespace
+
 namespace {
 struct QgPlan {
   int rt, ct, nq;
@@ -1064,6 +1178,19 @@ int qgemm_splits(int n, int mpad, int bits) {
   const int mt_all = mpad / 16;
   if (mt_all > 3) return n >= 16384 ? 2 : 4;
   return 4;
+}
+
+// K slices of the LM head: one, unless that leaves CUs without a workgroup
+// (small vocabularies), where the tail adds four slices as it reads them.
+// Measured on MI355X, 4096 x 4096 Q4: 35.7 us in one slice at 16 rows (16
+// workgroups), 28.4 at 45, 27.6 at 128 (128 workgroups).  One row (and two over
+// K <= 1024) takes the GEMV, one workgroup per column tile.
+int qgemm_head_splits(int n, int k, int rows, int bits) {
+  const int nb = k / 32, mt_all = (rows + 15) / 16;
+  if ((nb / 4) % 4 == 0 && (rows == 1 || (rows == 2 && k <= 1024))) return 1;
+  const QgPlan p = qg_plan(16 * mt_all, 1, bits, nb);
+  const int per = 4 * p.ct;
+  return (n / 16 + per - 1) / per * ((mt_all + p.rt - 1) / p.rt) < 256 ? 4 : 1;
 }
 
 // Launch arguments of one projection and the chunking choices made for it.
@@ -1142,6 +1269,8 @@ hipError_t launch_qgemm_form(hipStream_t st, const QTensor& w, const ActBuf& x, 
   // only on matrices up to 4M weights (Qwen3-0.6B down 4.3 vs 4.8).  Quarters
   // that are not whole 4-block groups (K = 640: Gemma-3-270M) stay on the tile,
   // whose preloaded chains were faster there (config1 0.750 vs 0.760 ms/step).
+  if (form == QG_FORM_AUTO && qgemm_res_serves(w, x.mpad, m_rows, splits))
+    return launch_qgemm_res(st, w, x, m_rows, y, ldy, slice_stride);
   if (form == QG_FORM_AUTO && x.mpad == 16 && m_rows <= 4) {
     if (m_rows == 1 && w.k >= 8192) {
       if (launch_qgemv(st, w, x, m_rows, y, ldy, splits, slice_stride) == hipSuccess) return hipSuccess;
@@ -1198,6 +1327,10 @@ hipError_t launch_qgemm_actin(hipStream_t st, const QTensor& w, const ActIn& ain
     return hipErrorNotSupported;
   if (w.n % 16 || nb % 4 || (splits != 1 && splits != 2 && splits != 4) || (w.bits != 4 && w.bits != 8))
     return hipErrorNotSupported;
+  // two rows over a long K: 26.6 us here (every workgroup rebuilds its part of
+  // the activation from four slices), 13.4 + 4.5 us as k_qgemm_res after the
+  // activation launch (4096 x 14336 Q4)
+  if (qgemm_res_serves(w, mpad, m_rows, splits)) return hipErrorNotSupported;
   ActBuf x{};
   x.mpad = mpad;
   if (m_rows <= 4) {
@@ -3716,23 +3849,31 @@ int argmax_segments(int rows, int vocab) {
   return std::max(1, std::min(s, 64));
 }
 
-__global__ __launch_bounds__(256) void k_argmax_part(const float* __restrict__ logits, int vocab, int seg,
+// S > 1: the logits come as S head slices, whose sums (the canonical tree) are
+// also written to `out`; vocab is then a multiple of 4.
+template <int S>
+__global__ __launch_bounds__(256) void k_argmax_part(Slices logits, float* __restrict__ out, int vocab, int seg,
                                                      int32_t* __restrict__ cand) {
   __shared__ float sv[256];
   __shared__ int si[256];
-  const int s = blockIdx.x, row = blockIdx.y, S = gridDim.x, tid = threadIdx.x;
+  const int s = blockIdx.x, row = blockIdx.y, segs = gridDim.x, tid = threadIdx.x;
   const int lo = min(vocab, s * seg), hi = min(vocab, lo + seg);
-  const float* lr = logits + (size_t)row * vocab;
+  const size_t r0 = (size_t)row * vocab;
+  const float* lr = logits.p + r0;
   float bv = 0.0f;
   int bi = INT_MAX;
   if ((vocab & 3) == 0) {
     // seg is a multiple of 4: float4 chunks, four loads in flight per thread
     const int c0 = lo >> 2, n4 = (hi - lo) >> 2;
-    const f4* l4 = reinterpret_cast<const f4*>(lr) + c0;
     for (int cb = tid; cb < n4; cb += 4 * 256) {
       f4 v[4];
 #pragma unroll
-      for (int j = 0; j < 4; j++) v[j] = l4[min(cb + j * 256, n4 - 1)];
+      for (int j = 0; j < 4; j++) v[j] = sl_get<S>(logits, r0 + 4 * (size_t)(c0 + min(cb + j * 256, n4 - 1)));
+      if constexpr (S > 1) {
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          if (cb + j * 256 < n4) *reinterpret_cast<f4*>(out + r0 + 4 * (size_t)(c0 + cb + j * 256)) = v[j];
+      }
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         const int c = cb + j * 256;
@@ -3760,8 +3901,8 @@ __global__ __launch_bounds__(256) void k_argmax_part(const float* __restrict__ l
     __syncthreads();
   }
   if (tid == 0) {
-    cand[((size_t)row * S + s) * 2] = __builtin_bit_cast(int32_t, sv[0]);
-    cand[((size_t)row * S + s) * 2 + 1] = si[0];
+    cand[((size_t)row * segs + s) * 2] = __builtin_bit_cast(int32_t, sv[0]);
+    cand[((size_t)row * segs + s) * 2 + 1] = si[0];
   }
 }
 
@@ -3805,11 +3946,16 @@ __global__ __launch_bounds__(64) void k_argmax_final(const int32_t* __restrict__
   }
 }
 
-hipError_t launch_argmax_gather(hipStream_t st, const float* logits, int rows, int vocab,
+hipError_t launch_argmax_gather(hipStream_t st, Slices logits, float* out, int rows, int vocab,
                                 const float* emb, int d, int32_t* tok, float* r0, int32_t* cand) {
   const int S = argmax_segments(rows, vocab);
   const int seg = ((vocab + S - 1) / S + 3) & ~3;
-  hipLaunchKernelGGL(k_argmax_part, dim3(S, rows), dim3(256), 0, st, logits, vocab, seg, cand);
+  if (logits.n == 1)
+    hipLaunchKernelGGL(k_argmax_part<1>, dim3(S, rows), dim3(256), 0, st, logits, out, vocab, seg, cand);
+  else if (logits.n == 4 && out && vocab % 4 == 0)
+    hipLaunchKernelGGL(k_argmax_part<4>, dim3(S, rows), dim3(256), 0, st, logits, out, vocab, seg, cand);
+  else
+    return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_argmax_final, dim3(rows), dim3(64), 0, st, cand, S, emb, d, tok, r0);
   return hipGetLastError();
 }

@@ -202,10 +202,11 @@ struct rstr_decoder {
   rstr_pool* p = nullptr;
   int B = 0, pps = 0, maxpos = 0, split = 0, mpad = 0, kmax = 0, max_items = 0;
   int qd = 0, kvr = 0, nqkv = 0;
-  int s_qkv = 1, s_o = 1, s_gu = 1, s_down = 1;   // split-K slices per projection
+  int s_qkv = 1, s_o = 1, s_gu = 1, s_down = 1, s_head = 1;   // split-K slices per projection
   // device state / scratch
   float *r0 = nullptr, *xmid = nullptr, *o = nullptr, *yqkv = nullptr, *qr = nullptr;
   float *gu = nullptr, *logits = nullptr, *part = nullptr;
+  float* head = nullptr;                            // head slices (s_head > 1; logits are their sums)
   float *rope_cos = nullptr, *rope_sin = nullptr;   // [2][maxpos][hd/2]
   ActBuf act;
   ActBuf act_ff;                                    // down-projection input when gate/up fuses the activation
@@ -991,7 +992,7 @@ static void decoder_free(rstr_decoder* d) {
   hipSetDevice(d->m->s->device);
   if (d->graph) hipGraphExecDestroy(d->graph);
   for (void* q : {(void*)d->r0, (void*)d->xmid, (void*)d->o, (void*)d->yqkv, (void*)d->qr, (void*)d->gu,
-                  (void*)d->logits, (void*)d->part, (void*)d->rope_cos, (void*)d->rope_sin,
+                  (void*)d->logits, (void*)d->head, (void*)d->part, (void*)d->rope_cos, (void*)d->rope_sin,
                   (void*)d->act.q, (void*)d->act.s, (void*)d->act_ff.q, (void*)d->act_ff.s,
                   (void*)d->desc, (void*)d->lane_tab,
                   (void*)d->tokbuf, (void*)d->amax_cand, (void*)d->d_lanes, (void*)d->d_tokens,
@@ -1041,6 +1042,7 @@ static int decoder_open(rstr_model* m, rstr_pool* p, int32_t batch, int32_t pps,
   d->s_o = qgemm_splits(md.d_model, d->mpad, md.weight_bits);
   d->s_gu = qgemm_splits(2 * md.d_ff, d->mpad, md.weight_bits);
   d->s_down = qgemm_splits(md.d_model, d->mpad, md.weight_bits);
+  d->s_head = qgemm_head_splits(md.vocab, md.d_model, batch, md.weight_bits);
   const int s_d = std::max(d->s_o, d->s_down);
   int64_t max_pos_tokens = std::min<int64_t>((int64_t)pps * p->page_size, (int64_t)maxpos + 1);
   int64_t splits = (max_pos_tokens + split - 1) / split + 1;
@@ -1064,6 +1066,7 @@ static int decoder_open(rstr_model* m, rstr_pool* p, int32_t batch, int32_t pps,
   d->fuse_act = qgemm_act_fused(md.d_ff, d->mpad);
   if (!d->fuse_act) A(dmalloc(&d->gu, (size_t)d->s_gu * batch * 2 * md.d_ff));
   if (head_tail) A(dmalloc(&d->logits, (size_t)batch * md.vocab));
+  if (head_tail && d->s_head > 1) A(dmalloc(&d->head, (size_t)d->s_head * batch * md.vocab));
   A(dmalloc(&d->part, (size_t)d->max_items * G * attn_part_floats(md.head_dim)));
   A(dmalloc(&d->rope_cos, (size_t)2 * maxpos * half));
   A(dmalloc(&d->rope_sin, (size_t)2 * maxpos * half));
@@ -1440,10 +1443,12 @@ static hipError_t enqueue_step(rstr_decoder* d, hipStream_t st, Prof* prof, bool
   }
   if (!d->head_tail) return e;
   run(RSTR_K_HEAD, [&] {
-    return launch_qgemm(st, d->m->head, d->act, B, d->logits, md.vocab, 1, (size_t)B * md.vocab);
+    return launch_qgemm(st, d->m->head, d->act, B, d->s_head > 1 ? d->head : d->logits, md.vocab, d->s_head,
+                        (size_t)B * md.vocab);
   });
   run(RSTR_K_TAIL, [&] {
-    return launch_argmax_gather(st, d->logits, B, md.vocab, d->m->emb, dm, d->tokbuf, d->r0, d->amax_cand);
+    return launch_argmax_gather(st, Slices{d->s_head > 1 ? d->head : d->logits, d->s_head, (size_t)B * md.vocab},
+                                d->logits, B, md.vocab, d->m->emb, dm, d->tokbuf, d->r0, d->amax_cand);
   });
   return e;
 }
@@ -1835,7 +1840,7 @@ extern "C" int rstr_tail_run(rstr_session* s, int32_t rows, int32_t vocab, int32
   if (e == hipSuccess) e = dmalloc(&dc, (size_t)2 * rows * argmax_segments(rows, vocab));
   if (e == hipSuccess) e = hipMemcpy(dl, logits, sizeof(float) * rows * vocab, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(de, emb, sizeof(float) * vocab * d, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = launch_argmax_gather(s->stream, dl, rows, vocab, de, d, dt, dr, dc);
+  if (e == hipSuccess) e = launch_argmax_gather(s->stream, Slices{dl, 1, 0}, nullptr, rows, vocab, de, d, dt, dr, dc);
   if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
   if (e == hipSuccess) e = hipMemcpy(tokens_out, dt, sizeof(int32_t) * rows, hipMemcpyDeviceToHost);
   if (e == hipSuccess) e = hipMemcpy(rows_out, dr, sizeof(float) * rows * d, hipMemcpyDeviceToHost);
