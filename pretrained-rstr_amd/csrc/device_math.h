@@ -165,24 +165,34 @@ __device__ __forceinline__ float xor_max(float v) {
   }
 }
 
-// xor butterfly: level m combines lanes i and i^m.  Because fp add commutes,
-// both lanes hold the same value and the result is the balanced pairwise tree
-// over lane order.
+// xor butterfly: level m combines lanes i and i^m.  Because fp add and max
+// commute, both lanes hold the same value and the result is the balanced
+// pairwise tree over lane order.  After levels 1 and 2 the four lanes of a quad
+// agree, so the mirrored lane of an 8-lane half row holds lane i^4's value, and
+// row_ror:8 is lane i^8: every level is a DPP operation or a lane swap (the
+// swizzle unit, an LDS round trip, took ~0.1 us a reduction in the row kernels).
+__device__ __forceinline__ float row_ror8_lane(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xF, 0xF, true));
+}
 __device__ __forceinline__ float wave_tree_sum(float v) {
   v = xor_add<1>(v);
   v = xor_add<2>(v);
-  v = xor_add<4>(v);
-  v = xor_add<8>(v);
+  v = v + half_mirror_lane(v);
+  v = v + row_ror8_lane(v);
   v = xor_add<16>(v);
   return xor_add<32>(v);
 }
-__device__ __forceinline__ float wave_max(float v) {
+// maximum over aligned groups of N lanes (N = 4, 8, 16, 32 or 64)
+template <int N>
+__device__ __forceinline__ float group_max(float v) {
   v = xor_max<1>(v);
   v = xor_max<2>(v);
-  v = xor_max<4>(v);
-  v = xor_max<8>(v);
-  v = xor_max<16>(v);
-  return xor_max<32>(v);
+  if constexpr (N >= 8) v = fmaxf(v, half_mirror_lane(v));
+  if constexpr (N >= 16) v = fmaxf(v, row_ror8_lane(v));
+  if constexpr (N >= 32) v = xor_max<16>(v);
+  if constexpr (N >= 64) v = xor_max<32>(v);
+  return v;
 }
+__device__ __forceinline__ float wave_max(float v) { return group_max<64>(v); }
 
 }  // namespace rstr

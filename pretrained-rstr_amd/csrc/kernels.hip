@@ -1441,9 +1441,7 @@ __device__ __forceinline__ float rms_scale(float ss, int n, float eps) {
 __device__ __forceinline__ void quant_store(f4 y, bool valid, int c, int row, int nb, int mpad,
                                             _Float16* __restrict__ Q, float* __restrict__ S) {
   float a = valid ? fmaxf(fmaxf(fabsf(y[0]), fabsf(y[1])), fmaxf(fabsf(y[2]), fabsf(y[3]))) : 0.0f;
-  a = fmaxf(a, xor_lane<1>(a));
-  a = fmaxf(a, xor_lane<2>(a));
-  a = fmaxf(a, xor_lane<4>(a));
+  a = group_max<8>(a);
   if (!valid) return;
   const float d = act_scale(a);
   const float id = (d != 0.0f) ? 1.0f / d : 0.0f;
@@ -1745,6 +1743,29 @@ hipError_t launch_qkv_post(hipStream_t st, Slices yqkv, int rows, int n_q, int n
 // Work item = (lane, kv head, history split of `split` tokens); items are
 // packed by a device-side lane table so ragged lanes cost only their pages.
 // ===========================================================================
+// Inclusive sum of v over the 1024 threads of a workgroup in thread order, and
+// the total: shuffles inside each wave, then the 16 wave sums.
+__device__ __forceinline__ int32_t block_scan(int32_t v, int32_t* s_w, int32_t& total) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int32_t t = __shfl_up(v, off, 64);
+    if (lane >= off) v += t;
+  }
+  __syncthreads();  // s_w may still be read by an earlier scan
+  if (lane == 63) s_w[wave] = v;
+  __syncthreads();
+  int32_t before = 0;
+  total = 0;
+#pragma unroll
+  for (int k = 0; k < 16; k++) {
+    const int32_t x = s_w[k];
+    if (k < wave) before += x;
+    total += x;
+  }
+  return v + before;
+}
+
 // Per-lane item table.  Item (lane b, kv head h, split k) covers the visible
 // tokens [max(lo, k*split), min(len, (k+1)*split)).  A split is full when it
 // holds `split` tokens; only a lane's first (window start) and last split can
@@ -1755,7 +1776,7 @@ __global__ __launch_bounds__(1024) void k_attn_prep(int batch, int split, int wi
   // tab: lo[B] k0[B] nsplit[B] base[B+1] fbase[B+1] pbase[B+1]; base, fbase
   // and pbase are exclusive prefix sums over lanes of the lane's items, full
   // items and partial items (integer sums: any order is exact)
-  __shared__ int32_t s_a[1024], s_f[1024], s_p[1024], s_h[RSTR_NCH];
+  __shared__ int32_t s_w[16], s_h[RSTR_NCH];
   int32_t* lo = tab;
   int32_t* k0 = tab + batch;
   int32_t* ns = tab + 2 * batch;
@@ -1792,32 +1813,18 @@ __global__ __launch_bounds__(1024) void k_attn_prep(int batch, int split, int wi
     }
     const int32_t va = b < batch ? n * n_kv : 0;
     const int32_t vf = b < batch ? f * n_kv : 0;
-    const int32_t vp = va - vf;
-    // inclusive Hillis-Steele scans over the 1024 lanes of this chunk
-    s_a[tid] = va;
-    s_f[tid] = vf;
-    s_p[tid] = vp;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-      const int32_t ta = tid >= off ? s_a[tid - off] : 0;
-      const int32_t tf = tid >= off ? s_f[tid - off] : 0;
-      const int32_t tp = tid >= off ? s_p[tid - off] : 0;
-      __syncthreads();
-      s_a[tid] += ta;
-      s_f[tid] += tf;
-      s_p[tid] += tp;
-      __syncthreads();
-    }
+    int32_t tot_a, tot_f;
+    const int32_t ia = block_scan(va, s_w, tot_a), jf = block_scan(vf, s_w, tot_f);
     if (b < batch) {
-      base[b] = carry_a + s_a[tid] - va;
-      fbase[b] = carry_f + s_f[tid] - vf;
-      pbase[b] = carry_p + s_p[tid] - vp;
+      base[b] = carry_a + ia - va;
+      fbase[b] = carry_f + jf - vf;
+      pbase[b] = carry_p + (ia - va) - (jf - vf);
     }
-    carry_a += s_a[1023];
-    carry_f += s_f[1023];
-    carry_p += s_p[1023];
-    __syncthreads();
+    carry_a += tot_a;
+    carry_f += tot_f;
+    carry_p += tot_a - tot_f;
   }
+  __syncthreads();  // the histogram is complete, the scans' sums are read
   // More items than the work list holds (descriptors the host validation
   // rejects): the step gets no attention work, so every output is 0, instead
   // of items written past the list.  carry_a is the same in every thread.
@@ -1837,17 +1844,11 @@ __global__ __launch_bounds__(1024) void k_attn_prep(int batch, int split, int wi
   // (inclusive scan over the reversed counts; thread r holds count NCH-1-r)
   static_assert(RSTR_NCH <= 1024, "one count per thread");
   const int32_t hv = tid < RSTR_NCH ? s_h[RSTR_NCH - 1 - tid] : 0;
-  s_a[tid] = hv;
-  __syncthreads();
-  for (int off = 1; off < RSTR_NCH; off <<= 1) {
-    const int32_t t = tid >= off ? s_a[tid - off] : 0;
-    __syncthreads();
-    s_a[tid] += t;
-    __syncthreads();
-  }
+  int32_t tot_h;
+  const int32_t ih = block_scan(hv, s_w, tot_h);
   if (tid < RSTR_NCH) {
     int32_t* boff = tab + attn_bucket_offset(batch);
-    boff[RSTR_NCH - 1 - tid] = s_a[tid] - hv;
+    boff[RSTR_NCH - 1 - tid] = ih - hv;
     boff[RSTR_NCH + (RSTR_NCH - 1 - tid)] = 0;  // fill cursor
   }
   if (tid == 0) {
@@ -1935,17 +1936,14 @@ struct AttnListArgs {
 };
 __global__ __launch_bounds__(1024) void k_attn_list(int batch, int split, int n_kv, int max_items,
                                                     const int32_t* __restrict__ lengths, AttnListArgs args) {
-  __shared__ int32_t s_a[1024], s_f[1024], s_p[1024], s_h[RSTR_NCH], s_cur[RSTR_NCH];
+  __shared__ int32_t s_w[16], s_h[RSTR_NCH], s_cur[RSTR_NCH];
   __shared__ int32_t s_lo[1024], s_k0[1024], s_ns[1024], s_len[1024], s_base[1025], s_fb[1025];
   const int gsel = blockIdx.x;
   const int window = args.window[gsel], R = args.R[gsel];
   int32_t* tab = args.tab[gsel];
   int4* items = args.items[gsel];
   const int tid = threadIdx.x;
-  for (int i = tid; i < RSTR_NCH; i += 1024) {
-    s_h[i] = 0;
-    s_cur[i] = 0;
-  }
+  for (int i = tid; i < RSTR_NCH; i += 1024) s_h[i] = 0;
   __syncthreads();
   // ---- lane tables (k_attn_prep, one chunk of lanes)
   const int b = tid;
@@ -1969,23 +1967,10 @@ __global__ __launch_bounds__(1024) void k_attn_list(int batch, int split, int n_
   }
   const int32_t va = b < batch ? n * n_kv : 0;
   const int32_t vf = b < batch ? f * n_kv : 0;
-  const int32_t vp = va - vf;
-  s_a[tid] = va;
-  s_f[tid] = vf;
-  s_p[tid] = vp;
-  __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {
-    const int32_t ta = tid >= off ? s_a[tid - off] : 0;
-    const int32_t tf = tid >= off ? s_f[tid - off] : 0;
-    const int32_t tp = tid >= off ? s_p[tid - off] : 0;
-    __syncthreads();
-    s_a[tid] += ta;
-    s_f[tid] += tf;
-    s_p[tid] += tp;
-    __syncthreads();
-  }
-  int32_t tot_a = s_a[1023], tot_f = s_f[1023], tot_p = s_p[1023];
-  int32_t base_b = s_a[tid] - va, fb_b = s_f[tid] - vf, pb_b = s_p[tid] - vp;
+  int32_t tot_a, tot_f;
+  const int32_t ia = block_scan(va, s_w, tot_a), jf = block_scan(vf, s_w, tot_f);
+  int32_t tot_p = tot_a - tot_f;
+  int32_t base_b = ia - va, fb_b = jf - vf, pb_b = base_b - fb_b;
   // more items than the list holds (descriptors the host validation rejects):
   // no attention work, every output 0 (as k_attn_prep)
   const bool over = tot_a > max_items;
@@ -2022,47 +2007,40 @@ __global__ __launch_bounds__(1024) void k_attn_list(int batch, int split, int n_
     tab[attn_ctl_offset(batch) + 1] = arm;
   }
   __syncthreads();
-  // partial items by decreasing chunk count: boff[c] = the partial items of
-  // all counts above c (exclusive suffix sum; thread r holds count NCH-1-r)
+  // partial items by decreasing chunk count: the cursor of count c starts at
+  // the partial items of all counts above c (exclusive suffix sum; thread r
+  // holds count NCH-1-r)
   static_assert(RSTR_NCH <= 1024, "one count per thread");
   const int32_t hv = tid < RSTR_NCH ? s_h[RSTR_NCH - 1 - tid] : 0;
-  s_a[tid] = hv;
+  int32_t tot_h;
+  const int32_t ih = block_scan(hv, s_w, tot_h);
+  if (tid < RSTR_NCH) s_cur[RSTR_NCH - 1 - tid] = ih - hv;
   __syncthreads();
-  for (int off = 1; off < RSTR_NCH; off <<= 1) {
-    const int32_t t = tid >= off ? s_a[tid - off] : 0;
-    __syncthreads();
-    s_a[tid] += t;
-    __syncthreads();
-  }
-  int32_t* s_boff = s_p;  // the last scan's array is free again
-  if (tid < RSTR_NCH) s_boff[RSTR_NCH - 1 - tid] = s_a[tid] - hv;
-  __syncthreads();
-  // ---- the work list (k_attn_items)
-  for (int i = tid; i < tot_a; i += 1024) {
-    int bl = 0, hi = batch;
-    while (hi - bl > 1) {
-      const int mid = (bl + hi) >> 1;
-      if (s_base[mid] <= i) bl = mid; else hi = mid;
+  // ---- the work list (k_attn_items), one wave per lane of the batch: its
+  // items' numbers follow from the lane alone (a search for the lane of every
+  // item cost ~1 us a thousand items)
+  const int wl = tid & 63;
+  for (int bl = __builtin_amdgcn_readfirstlane(tid >> 6); bl < batch; bl += 16) {
+    const int ns = s_ns[bl], n_it = ns * n_kv;
+    if (n_it == 0) continue;
+    const int ln = s_len[bl], lb = s_lo[bl], k0 = s_k0[bl], ib = s_base[bl], fb = s_fb[bl];
+    const int nf = (s_fb[bl + 1] - fb) / n_kv;
+    const bool first_partial = !(lb == k0 * split && min(ln, (k0 + 1) * split) - lb == split);
+    for (int rel = wl; rel < n_it; rel += 64) {
+      const int kvh = rel / ns;
+      const int sp = rel - kvh * ns;
+      const int k = k0 + sp;
+      const int t0 = max(lb, k * split), t1 = min(ln, (k + 1) * split);
+      const int before = (first_partial && sp > 0) ? 1 : 0;
+      int pos;
+      if (t1 - t0 == split) {
+        pos = fb + kvh * nf + (sp - before);
+      } else {
+        const int nch = (t1 - (t0 & ~15) + 15) >> 4;
+        pos = tot_f + atomicAdd(&s_cur[nch], 1);
+      }
+      items[pos] = int4{bl | (kvh << 20), t0, t1, ib + rel};
     }
-    const int ns = s_ns[bl];
-    const int rel = i - s_base[bl];
-    const int kvh = rel / ns;
-    const int sp = rel % ns;
-    const int ln = s_len[bl];
-    const int k = s_k0[bl] + sp;
-    const int t0 = max(s_lo[bl], k * split), t1 = min(ln, (k + 1) * split);
-    const int nf = (s_fb[bl + 1] - s_fb[bl]) / n_kv;
-    const int lb = s_lo[bl];
-    const bool first_partial = !(lb == s_k0[bl] * split && min(ln, (s_k0[bl] + 1) * split) - lb == split);
-    const int before = (first_partial && sp > 0) ? 1 : 0;
-    int pos;
-    if (t1 - t0 == split) {
-      pos = s_fb[bl] + kvh * nf + (sp - before);
-    } else {
-      const int nch = (t1 - (t0 & ~15) + 15) >> 4;
-      pos = tot_f + s_boff[nch] + atomicAdd(&s_cur[nch], 1);
-    }
-    items[pos] = int4{bl | (kvh << 20), t0, t1, i};
   }
 }
 
@@ -3690,8 +3668,7 @@ __global__ __launch_bounds__(64) void k_attn_merge(int batch, int n_q, int n_kv,
     float a = 0.0f;
 #pragma unroll
     for (int d = 0; d < DPL; d++) a = fmaxf(a, fabsf(O[d]));
-#pragma unroll
-    for (int m = 1; m < 32 / DPL; m <<= 1) a = fmaxf(a, __shfl_xor(a, m, 64));
+    a = group_max<32 / DPL>(a);
     const float dq = act_scale(a);
     const float id = (dq != 0.0f) ? 1.0f / dq : 0.0f;
     const int qd = n_q * HD, nb = qd >> 5;
@@ -3779,9 +3756,7 @@ __global__ __launch_bounds__(64) void k_attn_merge_wide(int batch, int n_q, int 
   if (out_f32) out_f32[((size_t)b * n_q + h) * HD + dim] = O;
   if (Q) {
     // 32-dim blocks: 32 lanes per block
-    float a = fabsf(O);
-#pragma unroll
-    for (int m = 1; m < 32; m <<= 1) a = fmaxf(a, __shfl_xor(a, m, 64));
+    const float a = group_max<32>(fabsf(O));
     const float dq = act_scale(a);
     const float id = (dq != 0.0f) ? 1.0f / dq : 0.0f;
     const int qd = n_q * HD, nb = qd >> 5;
