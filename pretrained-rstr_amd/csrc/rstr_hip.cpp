@@ -18,6 +18,7 @@
 #include <cstdio>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -160,9 +161,10 @@ struct rstr_pool {
   void* attn_dev = nullptr;
   void* attn_host = nullptr;
   size_t attn_dev_bytes = 0, attn_host_bytes = 0;
+  std::mutex attn_mu;  // held by the call that uses them
 };
 // What a pool keeps for the isolated attention between calls, per buffer;
-// larger calls allocate and free their own.
+// larger calls, and calls that find the buffers in use, allocate and free their own.
 static constexpr size_t kAttnKeep = (size_t)128 << 20;
 
 struct rstr_transfer {
@@ -2084,7 +2086,8 @@ extern "C" int rstr_attention_run(rstr_pool* p, int32_t layer, int32_t batch, in
   if (rc) return rc;
   hipStream_t st = s->stream;
   // grow what the pool keeps (nothing of an earlier call is still running), or
-  // take memory for this call alone
+  // take memory for this call alone; what is kept is given back before more is
+  // asked for, so a call fits wherever it fits without it
   const size_t in_bytes = bk.o_out, host_bytes = std::max(in_bytes, bk.qb);
   struct Own {
     void *dev = nullptr, *host = nullptr;
@@ -2093,30 +2096,35 @@ extern "C" int rstr_attention_run(rstr_pool* p, int32_t layer, int32_t batch, in
       if (host) hipHostFree(host);
     }
   } own;
-  void *dev = p->attn_dev, *host = p->attn_host;
-  if (bk.total > p->attn_dev_bytes) {
-    void* n = nullptr;
-    HIPCHK(s, hipMalloc(&n, bk.total));
-    if (bk.total <= kAttnKeep) {
-      if (p->attn_dev) hipFree(p->attn_dev);
-      p->attn_dev = n;
+  std::unique_lock<std::mutex> kept(p->attn_mu, std::try_to_lock);
+  void *dev = kept ? p->attn_dev : nullptr, *host = kept ? p->attn_host : nullptr;
+  if (!kept || bk.total > p->attn_dev_bytes) {
+    if (kept && p->attn_dev) {
+      hipFree(p->attn_dev);
+      p->attn_dev = nullptr;
+      p->attn_dev_bytes = 0;
+    }
+    HIPCHK(s, hipMalloc(&dev, bk.total));
+    if (kept && bk.total <= kAttnKeep) {
+      p->attn_dev = dev;
       p->attn_dev_bytes = bk.total;
     } else {
-      own.dev = n;
+      own.dev = dev;
     }
-    dev = n;
   }
-  if (host_bytes > p->attn_host_bytes) {
-    void* n = nullptr;
-    HIPCHK(s, hipHostMalloc(&n, host_bytes));
-    if (host_bytes <= kAttnKeep) {
-      if (p->attn_host) hipHostFree(p->attn_host);
-      p->attn_host = n;
+  if (!kept || host_bytes > p->attn_host_bytes) {
+    if (kept && p->attn_host) {
+      hipHostFree(p->attn_host);
+      p->attn_host = nullptr;
+      p->attn_host_bytes = 0;
+    }
+    HIPCHK(s, hipHostMalloc(&host, host_bytes));
+    if (kept && host_bytes <= kAttnKeep) {
+      p->attn_host = host;
       p->attn_host_bytes = host_bytes;
     } else {
-      own.host = n;
+      own.host = host;
     }
-    host = n;
   }
   char *hb = static_cast<char*>(host), *db = static_cast<char*>(dev);
   std::memcpy(hb + bk.o_q, q, bk.qb);

@@ -2,6 +2,8 @@
 calls that grow, fit in and exceed what is kept give the same bits, on two pools
 of one session in turn.  The reference of each lane is the same lane in a call
 of its own through the allocation-free entry."""
+from concurrent.futures import ThreadPoolExecutor
+
 import numpy as np
 import pytest
 
@@ -31,3 +33,24 @@ def test_calls_of_any_size_share_the_kept_blocks():
                 for b in (0, lanes // 2, lanes - 1):
                     want = p.attention(0, q[b:b + 1], table[b:b + 1], lengths[b:b + 1], split=split, static=True)
                     assert np.array_equal(got[b].view(np.uint32), want[0].view(np.uint32)), (lanes, split, b)
+
+
+@pytest.mark.gpu
+def test_a_call_beside_another_takes_its_own_blocks():
+    print("case attention beside attention", flush=True)
+    cfg = dict(configs.TINY_QWEN, n_layers=1, n_q=8, n_kv=1, head_dim=128, vocab=512)
+    ps, pages = 16, 64
+    rng = np.random.default_rng(4)
+    with hip.Session(0) as s:
+        p = hip.Pool(hip.Model(s, cfg, seed=1), ps, pages)
+        p.fill_synthetic(np.arange(pages), seed=3)
+        args = []
+        for lanes in (5, 9):
+            q = rng.standard_normal((lanes, 8, 128)).astype(np.float32)
+            table = np.stack([rng.permutation(pages) for _ in range(lanes)]).astype(np.int32)
+            args.append((q, table, rng.integers(1, pages * ps + 1, lanes).astype(np.int32)))
+        want = [p.attention(0, *a, split=64, static=True) for a in args]
+        with ThreadPoolExecutor(2) as threads:
+            calls = [(i, threads.submit(p.attention, 0, *args[i], split=64)) for _ in range(20) for i in (0, 1)]
+            for i, c in calls:
+                assert np.array_equal(c.result().view(np.uint32), want[i].view(np.uint32)), i
