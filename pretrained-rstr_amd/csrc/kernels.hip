@@ -1170,14 +1170,19 @@ QgPlan qg_plan(int mpad, int splits, int bits, int nb) {
 }
 }  // namespace
 
-// K slices for a projection of width n at this batch: one slice where the
-// output is large and read once (gate/up at small batches, the head), two for
-// wide projections, four where few column blocks would leave CUs idle.
+// K slices for a projection of width n at this batch: two for wide projections
+// and where two leave four 64 x 64 workgroups to every CU, four where fewer
+// column blocks would leave CUs idle.  Each slice is written and read back by
+// the row kernel behind it, so two halve that traffic, but a wave's chain is
+// twice as long.  Measured on MI355X, us for four layers at four slices and at
+// two for qkv, o and down: Llama-3-8B 512 rows (1536 and 1024 workgroups at
+// two) 1990 and 1931, Q8 2259 and 2154; 256 rows (768, 512) 1120 and 1139, 160
+// rows (576, 384) 886 and 948; Gemma-3-270M 512 rows (384, 160) 425 and 437.
 int qgemm_splits(int n, int mpad, int bits) {
   (void)bits;
   const int mt_all = mpad / 16;
-  if (mt_all > 3) return n >= 16384 ? 2 : 4;
-  return 4;
+  const int wgs = (n + 63) / 64 * ((mt_all + 3) / 4) * 2;
+  return mt_all > 3 && (n >= 16384 || wgs >= 1024) ? 2 : 4;
 }
 
 // K slices of the LM head: one, unless that leaves CUs without a workgroup

@@ -106,3 +106,18 @@ def test_infinite_values_reach_only_the_rows_that_see_them(hd, window):
             x, y = a.view(np.float16), b.view(np.float16)
             assert np.array_equal(np.isnan(x), np.isnan(y)), i
             assert np.array_equal(a[~np.isnan(x)], b[~np.isnan(x)]), i
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("d_model,d_ff,n_q,n_kv", [(640, 256, 16, 8), (4096, 512, 4, 2)])
+def test_large_tiles_in_two_slices_match_the_oracle(d_model, d_ff, n_q, n_kv, bits):
+    """At 449 rows a 4096-wide projection runs in two K slices: the qkv
+    projection over K = 640 (quarters of five blocks), or o and down."""
+    print("case two slices", d_model, bits, flush=True)
+    cfg = dict(_cfg(128, n_q, n_kv, 0), n_layers=2, d_model=d_model, d_ff=d_ff, weight_bits=bits)
+    out, want = _tile(cfg, 449, 20, 0, 16, 256)
+    for rows_out, pages in out:
+        assert np.isfinite(rows_out).all()
+        for i, (a, b) in enumerate(zip(pages, want)):
+            assert np.array_equal(a, b), i
