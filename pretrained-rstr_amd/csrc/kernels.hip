@@ -3072,9 +3072,29 @@ __device__ __forceinline__ void wait_vm(int n) {
   }
 }
 
+// minimum and maximum over aligned groups of 16 lanes, all in DPP: after the
+// quad levels the mirrored lanes of a half row and of a row hold the values of
+// lanes i^4 and i^8
+template <int CTRL>
+__device__ __forceinline__ int dpp_i(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true);
+}
+__device__ __forceinline__ int row_min(int v) {
+  v = min(v, dpp_i<0xB1>(v));
+  v = min(v, dpp_i<0x4E>(v));
+  v = min(v, dpp_i<0x141>(v));
+  return min(v, dpp_i<0x140>(v));
+}
+__device__ __forceinline__ int row_max(int v) {
+  v = max(v, dpp_i<0xB1>(v));
+  v = max(v, dpp_i<0x4E>(v));
+  v = max(v, dpp_i<0x141>(v));
+  return max(v, dpp_i<0x140>(v));
+}
+
 template <int HD, int G>
 __global__ __launch_bounds__(256, HD == 128 ? 3 : 2) void k_attn_tile(
-    int batch, int n_kv, int page_size, int ps_shift, int pps, int split, int window, float scale,
+    int batch, int n_kv, int page_size, int ps_shift, int pps, int split, float scale,
     const float* __restrict__ q, const uint16_t* __restrict__ kp, const uint16_t* __restrict__ vp,
     const int32_t* __restrict__ page_table, const int32_t* __restrict__ lengths,
     const int32_t* __restrict__ tab, float* __restrict__ part) {
@@ -3084,266 +3104,281 @@ __global__ __launch_bounds__(256, HD == 128 ? 3 : 2) void k_attn_tile(
   constexpr int RV = 8 / H;         // V chunks in a wave's LDS
   constexpr int PF = attn_part_floats(HD);
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   u32x4* ring = reinterpret_cast<u32x4*>(smem) + wave * 512;                    // this wave's 8 KB
   float* red = reinterpret_cast<float*>(smem + 32768);                          // [wave][16] maxima
   f4* sc = reinterpret_cast<f4*>(red + 64);                                     // [chunk][lane] scores
-  const int i = lane & 15, g = lane >> 4;
-  const int kvh = blockIdx.x, r0 = blockIdx.y * RPT, s = blockIdx.z;
+  const int kvh = blockIdx.x, r0 = blockIdx.y * RPT;
   const int kvr = n_kv * HD;
-  const int ts = s * split, te = ts + split;
-  // the visible part [a, e) of this split for the lane's row; a row without items has none
-  const int row = r0 + i / G, head = i % G;
-  int a = INT_MAX, e = INT_MIN;
-  if (row < batch) {
-    const int len = lengths[row], ns = tab[2 * batch + row];
-    const int a0 = max(window > 0 ? max(0, len - window) : 0, ts), e0 = min(len, te);
-    if (a0 < e0 && ns > 0) { a = a0; e = e0; }
-  }
-  int lo = a, hi = e, flo = a, fhi = e;  // tokens some row sees, tokens every row sees
-#pragma unroll
-  for (int m = 1; m < 16; m <<= 1) {
-    lo = min(lo, __shfl_xor(lo, m, 64));
-    hi = max(hi, __shfl_xor(hi, m, 64));
-    flo = max(flo, __shfl_xor(flo, m, 64));
-    fhi = min(fhi, __shfl_xor(fhi, m, 64));
-  }
-  lo = uni(lo);
-  hi = uni(hi);
-  flo = uni(flo);
-  fhi = uni(fhi);
-  if (lo >= hi) return;
-  const int T0 = lo & ~15, nch = (hi - T0 + 15) >> 4;
-  auto whole = [&](int c) { return T0 + 16 * c >= flo && T0 + 16 * c + 16 <= fhi; };  // every row sees all of chunk c
-  // page of each chunk, in lane (page index)
-  const int pg0 = T0 >> ps_shift, npg = ((T0 + (nch - 1) * 16) >> ps_shift) - pg0 + 1;
-  int pgv[2];
-#pragma unroll
-  for (int k = 0; k < 2; k++) pgv[k] = lane + 64 * k < npg ? page_table[(size_t)r0 * pps + pg0 + 64 * k + lane] : 0;
-  const uint32_t row_bytes = (uint32_t)kvr * 2u;
-  const uint32_t page_bytes = (uint32_t)page_size * row_bytes;
-  auto chunk_base = [&](const uint16_t* slab, int c) -> const char* {
-    const int tb = T0 + c * 16, pi = (tb >> ps_shift) - pg0;
-    int page = __builtin_amdgcn_readlane(pgv[0], pi & 63);
-    if (pi >= 64) page = __builtin_amdgcn_readlane(pgv[1], pi & 63);
-    return reinterpret_cast<const char*>(slab + kvh * HD) + (uint64_t)(uint32_t)page * page_bytes +
-           (uint32_t)(tb & (page_size - 1)) * row_bytes;
-  };
-  // K: one half of a chunk in 4 KB, piece p of row r at slot p ^ r
-  auto issue_k = [&](int n) {
-    const char* base = chunk_base(kp, wave + 4 * (n / H)) + (n % H) * 256;
-    u32x4* dst = ring + (n & 1) * 256;
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int r = u * 4 + g;
-      __builtin_amdgcn_global_load_lds(reinterpret_cast<const void*>(base + (uint32_t)r * row_bytes + (uint32_t)(i ^ r) * 16u),
-                                       RSTR_LDS_PTR(dst + u * 64), 16, 0, 0);
-    }
-  };
-  // V: this wave's dims of a chunk, rows of 64*H bytes
-  auto issue_v = [&](int c) {
-    const char* base = chunk_base(vp, c) + wave * (HD / 2);
-    u32x4* dst = ring + (c % RV) * (64 * H);
-#pragma unroll
-    for (int u = 0; u < H; u++) {
-      const int un = u * 64 + lane;
-      __builtin_amdgcn_global_load_lds(
-          reinterpret_cast<const void*>(base + (uint32_t)(un / (4 * H)) * row_bytes + (uint32_t)(un % (4 * H)) * 16u),
-          RSTR_LDS_PTR(dst + u * 64), 16, 0, 0);
-    }
-  };
-  // the queries: lane (block g, pair i) holds slices 4g..4g+3 of pair i
-  float qv[H][4][8];
+  // the lane's row: its visible range [v0, len), and the record index of its
+  // split s as rec0 + s; a row without items sees nothing
+  int v0, len, rec0, sa, sb;
   {
-    const float* qr = q + ((size_t)min(row, batch - 1) * (n_kv * G) + kvh * G + head) * HD;
-#pragma unroll
-    for (int h = 0; h < H; h++)
-#pragma unroll
-      for (int sl = 0; sl < 4; sl++) {
-        const f4 x = *reinterpret_cast<const f4*>(qr + h * 128 + (4 * g + sl) * 8);
-        const f4 y = *reinterpret_cast<const f4*>(qr + h * 128 + (4 * g + sl) * 8 + 4);
-#pragma unroll
-        for (int d = 0; d < 4; d++) { qv[h][sl][d] = x[d]; qv[h][sl][4 + d] = y[d]; }
-      }
+    const int r = r0 + (threadIdx.x & 15) / G, rr = min(r, batch - 1);
+    const int rl = lengths[rr], rk = tab[batch + rr], rn = tab[2 * batch + rr], rb = tab[3 * batch + rr];
+    const bool live = r < batch && rn > 0;
+    v0 = tab[rr];
+    len = live ? rl : 0;
+    rec0 = rb + kvh * rn - rk;
+    sa = live ? rk : INT_MAX;
+    sb = live ? rk + rn - 1 : -1;
   }
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // page ids and queries have arrived
-  __asm__ __volatile__("" ::: "memory");
-  const int nk = nch > wave ? (nch - wave + 3) >> 2 : 0, npos = nk * H;  // this wave's K chunks
-  if (npos > 0) issue_k(0);
-  if (npos > 1) issue_k(1);
-  if (npos == 0)
-    for (int c = 0; c < RV && c < nch; c++) issue_v(c);
-  const f16v zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-  float mx = -__builtin_inff();
-  const int tr = 4 * (i & 3) + (i >> 2);  // K row of the A operand's row i
-  for (int n = 0; n < nk; n++) {
-    const int c = wave + 4 * n, tb = T0 + c * 16;
-    f16v acc[4];
+  sa = uni(row_min(sa));  // splits of the group's rows
+  sb = uni(row_max(sb));
+  // Workgroup z takes the group's split z; where the launch has fewer (Z) than
+  // the group's splits, those from Z on go to the first half of the workgroups
+  // in turn, and the second half, one split each, fills the launch's end.
+  const int z = blockIdx.z, Z = gridDim.z, first = (Z + 1) >> 1;
+  for (int s = sa + z; s <= sb; s += s - sa < Z ? (z < first ? Z : INT_MAX / 2) : first) {
+    // opaque, so that the lane's addresses are formed anew for each split: kept
+    // over the loop they take 20 more registers and spill
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63;
+    const int i = lane & 15, g = lane >> 4;
+    const int row = r0 + i / G, head = i % G;
+    const int ts = s * split, te = ts + split;
+    // the visible part [a, e) of this split for the lane's row
+    int a = max(v0, ts), e = min(len, te);
+    if (a >= e) {
+      a = INT_MAX;
+      e = INT_MIN;
+    }
+    // tokens some row sees, tokens every row sees
+    const int lo = uni(row_min(a)), hi = uni(row_max(e)), flo = uni(row_max(a)), fhi = uni(row_min(e));
+    if (lo >= hi) continue;
+    const int T0 = lo & ~15, nch = (hi - T0 + 15) >> 4;
+    auto whole = [&](int c) { return T0 + 16 * c >= flo && T0 + 16 * c + 16 <= fhi; };  // every row sees all of chunk c
+    // page of each chunk, in lane (page index)
+    const int pg0 = T0 >> ps_shift, npg = ((T0 + (nch - 1) * 16) >> ps_shift) - pg0 + 1;
+    int pgv[2];
 #pragma unroll
-    for (int h = 0; h < H; h++) {
-      const int p = n * H + h;
-      if (p + 1 < npos) __builtin_amdgcn_s_waitcnt(0x0F74);  // vmcnt(4): position p has landed
-      else __builtin_amdgcn_s_waitcnt(0x0F70);
-      __asm__ __volatile__("" ::: "memory");
-      const u32x4* buf = ring + (p & 1) * 256;
-      h8 kv[4];
+    for (int k = 0; k < 2; k++) pgv[k] = lane + 64 * k < npg ? page_table[(size_t)r0 * pps + pg0 + 64 * k + lane] : 0;
+    const uint32_t row_bytes = (uint32_t)kvr * 2u;
+    const uint32_t page_bytes = (uint32_t)page_size * row_bytes;
+    auto chunk_base = [&](const uint16_t* slab, int c) -> const char* {
+      const int tb = T0 + c * 16, pi = (tb >> ps_shift) - pg0;
+      int page = __builtin_amdgcn_readlane(pgv[0], pi & 63);
+      if (pi >= 64) page = __builtin_amdgcn_readlane(pgv[1], pi & 63);
+      return reinterpret_cast<const char*>(slab + kvh * HD) + (uint64_t)(uint32_t)page * page_bytes +
+             (uint32_t)(tb & (page_size - 1)) * row_bytes;
+    };
+    // K: one half of a chunk in 4 KB, piece p of row r at slot p ^ r
+    auto issue_k = [&](int n) {
+      const char* base = chunk_base(kp, wave + 4 * (n / H)) + (n % H) * 256;
+      u32x4* dst = ring + (n & 1) * 256;
 #pragma unroll
-      for (int sl = 0; sl < 4; sl++) kv[sl] = __builtin_bit_cast(h8, buf[tr * 16 + ((4 * g + sl) ^ tr)]);
-      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the slot is free
-      __asm__ __volatile__("" ::: "memory");
-      if (p + 2 < npos) issue_k(p + 2);
-      else if (p + 1 == npos)
-        for (int v = 0; v < RV && v < nch; v++) issue_v(v);
-      // conversions of two slices, then their instructions (interleaved, each
-      // conversion stalls the matrix instruction that reads it)
+      for (int u = 0; u < 4; u++) {
+        const int r = u * 4 + g;
+        __builtin_amdgcn_global_load_lds(reinterpret_cast<const void*>(base + (uint32_t)r * row_bytes + (uint32_t)(i ^ r) * 16u),
+                                         RSTR_LDS_PTR(dst + u * 64), 16, 0, 0);
+      }
+    };
+    // V: this wave's dims of a chunk, rows of 64*H bytes
+    auto issue_v = [&](int c) {
+      const char* base = chunk_base(vp, c) + wave * (HD / 2);
+      u32x4* dst = ring + (c % RV) * (64 * H);
 #pragma unroll
-      for (int s2 = 0; s2 < 4; s2 += 2) {
-        float kf[2][8];
+      for (int u = 0; u < H; u++) {
+        const int un = u * 64 + lane;
+        __builtin_amdgcn_global_load_lds(
+            reinterpret_cast<const void*>(base + (uint32_t)(un / (4 * H)) * row_bytes + (uint32_t)(un % (4 * H)) * 16u),
+            RSTR_LDS_PTR(dst + u * 64), 16, 0, 0);
+      }
+    };
+    // the queries: lane (block g, pair i) holds slices 4g..4g+3 of pair i
+    float qv[H][4][8];
+    {
+      const float* qr = q + ((size_t)min(row, batch - 1) * (n_kv * G) + kvh * G + head) * HD;
 #pragma unroll
-        for (int sl = 0; sl < 2; sl++)
+      for (int h = 0; h < H; h++)
 #pragma unroll
-          for (int d = 0; d < 8; d++) kf[sl][d] = (float)kv[s2 + sl][d];
-        __builtin_amdgcn_sched_barrier(0);
+        for (int sl = 0; sl < 4; sl++) {
+          const f4 x = *reinterpret_cast<const f4*>(qr + h * 128 + (4 * g + sl) * 8);
+          const f4 y = *reinterpret_cast<const f4*>(qr + h * 128 + (4 * g + sl) * 8 + 4);
 #pragma unroll
-        for (int d = 0; d < 8; d++)
+          for (int d = 0; d < 4; d++) { qv[h][sl][d] = x[d]; qv[h][sl][4 + d] = y[d]; }
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // page ids and queries have arrived
+    __asm__ __volatile__("" ::: "memory");
+    const int nk = nch > wave ? (nch - wave + 3) >> 2 : 0, npos = nk * H;  // this wave's K chunks
+    if (npos > 0) issue_k(0);
+    if (npos > 1) issue_k(1);
+    if (npos == 0)
+      for (int c = 0; c < RV && c < nch; c++) issue_v(c);
+    const f16v zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    float mx = -__builtin_inff();
+    const int tr = 4 * (i & 3) + (i >> 2);  // K row of the A operand's row i
+    for (int n = 0; n < nk; n++) {
+      const int c = wave + 4 * n, tb = T0 + c * 16;
+      f16v acc[4];
+#pragma unroll
+      for (int h = 0; h < H; h++) {
+        const int p = n * H + h;
+        if (p + 1 < npos) __builtin_amdgcn_s_waitcnt(0x0F74);  // vmcnt(4): position p has landed
+        else __builtin_amdgcn_s_waitcnt(0x0F70);
+        __asm__ __volatile__("" ::: "memory");
+        const u32x4* buf = ring + (p & 1) * 256;
+        h8 kv[4];
+#pragma unroll
+        for (int sl = 0; sl < 4; sl++) kv[sl] = __builtin_bit_cast(h8, buf[tr * 16 + ((4 * g + sl) ^ tr)]);
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the slot is free
+        __asm__ __volatile__("" ::: "memory");
+        if (p + 2 < npos) issue_k(p + 2);
+        else if (p + 1 == npos)
+          for (int v = 0; v < RV && v < nch; v++) issue_v(v);
+        // conversions of two slices, then their instructions (interleaved, each
+        // conversion stalls the matrix instruction that reads it)
+#pragma unroll
+        for (int s2 = 0; s2 < 4; s2 += 2) {
+          float kf[2][8];
 #pragma unroll
           for (int sl = 0; sl < 2; sl++)
-            acc[s2 + sl] = __builtin_amdgcn_mfma_f32_16x16x1f32(kf[sl][d], qv[h][s2 + sl][d],
-                                                                h == 0 && d == 0 ? zero : acc[s2 + sl], 0, 0, 0);
+#pragma unroll
+            for (int d = 0; d < 8; d++) kf[sl][d] = (float)kv[s2 + sl][d];
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int d = 0; d < 8; d++)
+#pragma unroll
+            for (int sl = 0; sl < 2; sl++)
+              acc[s2 + sl] = __builtin_amdgcn_mfma_f32_16x16x1f32(kf[sl][d], qv[h][s2 + sl][d],
+                                                                  h == 0 && d == 0 ? zero : acc[s2 + sl], 0, 0, 0);
+        }
       }
-    }
-    f4 sv;
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      float t[4];
-#pragma unroll
-      for (int sl = 0; sl < 4; sl++) t[sl] = (acc[sl][r] + acc[sl][8 + r]) + (acc[sl][4 + r] + acc[sl][12 + r]);
-      sv[r] = ((t[0] + t[2]) + (t[1] + t[3])) * scale;
-    }
-    sc[c * 64 + lane] = sv;
-    if (whole(c)) {
-      mx = fmaxf(fmaxf(mx, fmaxf(sv[0], sv[1])), fmaxf(sv[2], sv[3]));
-    } else {
+      f4 sv;
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const int tk = tb + 4 * r + g;
-        mx = fmaxf(mx, tk >= a && tk < e ? sv[r] : -__builtin_inff());
+        float t[4];
+#pragma unroll
+        for (int sl = 0; sl < 4; sl++) t[sl] = (acc[sl][r] + acc[sl][8 + r]) + (acc[sl][4 + r] + acc[sl][12 + r]);
+        sv[r] = ((t[0] + t[2]) + (t[1] + t[3])) * scale;
+      }
+      sc[c * 64 + lane] = sv;
+      if (whole(c)) {
+        mx = fmaxf(fmaxf(mx, fmaxf(sv[0], sv[1])), fmaxf(sv[2], sv[3]));
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int tk = tb + 4 * r + g;
+          mx = fmaxf(mx, tk >= a && tk < e ? sv[r] : -__builtin_inff());
+        }
       }
     }
-  }
-  // ---- the split's maxima, then the softmax numerators ------------------------------
-  mx = xor_max<32>(xor_max<16>(mx));
-  if (g == 0) red[wave * 16 + i] = mx;
-  __builtin_amdgcn_s_waitcnt(0xC07F);
-  __asm__ __volatile__("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  __asm__ __volatile__("" ::: "memory");
-  mx = fmaxf(fmaxf(red[i], red[16 + i]), fmaxf(red[32 + i], red[48 + i]));
-  for (int c = wave; c < nch; c += 4) {
-    f4 p = sc[c * 64 + lane];
+    // ---- the split's maxima, then the softmax numerators ------------------------------
+    mx = xor_max<32>(xor_max<16>(mx));
+    if (g == 0) red[wave * 16 + i] = mx;
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __asm__ __volatile__("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    __asm__ __volatile__("" ::: "memory");
+    mx = fmaxf(fmaxf(red[i], red[16 + i]), fmaxf(red[32 + i], red[48 + i]));
+    for (int c = wave; c < nch; c += 4) {
+      f4 p = sc[c * 64 + lane];
 #pragma unroll
-    for (int r = 0; r < 4; r++) p[r] = dexp(p[r] - mx);
-    if (!whole(c)) {
+      for (int r = 0; r < 4; r++) p[r] = dexp(p[r] - mx);
+      if (!whole(c)) {
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int tk = T0 + c * 16 + 4 * r + g;
-        p[r] = tk >= a && tk < e ? p[r] : 0.0f;
+        for (int r = 0; r < 4; r++) {
+          const int tk = T0 + c * 16 + 4 * r + g;
+          p[r] = tk >= a && tk < e ? p[r] : 0.0f;
+        }
       }
+      sc[c * 64 + lane] = p;
     }
-    sc[c * 64 + lane] = p;
-  }
-  __builtin_amdgcn_s_waitcnt(0xC07F);
-  __asm__ __volatile__("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  __asm__ __volatile__("" ::: "memory");
-  // ---- PV -----------------------------------------------------------------------------
-  typedef _Float16 hv __attribute__((ext_vector_type(VD)));
-  f16v o[VD];
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __asm__ __volatile__("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    __asm__ __volatile__("" ::: "memory");
+    // ---- PV -----------------------------------------------------------------------------
+    typedef _Float16 hv __attribute__((ext_vector_type(VD)));
+    f16v o[VD];
 #pragma unroll
-  for (int d = 0; d < VD; d++) o[d] = zero;
-  float l = 0.0f;
-  bool special = false;  // this lane took non-finite V out of a chunk
-  auto load = [&](int c, hv (&vv)[4], f4& p) {
-    const _Float16* buf = reinterpret_cast<const _Float16*>(ring + (c % RV) * (64 * H));
+    for (int d = 0; d < VD; d++) o[d] = zero;
+    float l = 0.0f;
+    bool special = false;  // this lane took non-finite V out of a chunk
+    auto load = [&](int c, hv (&vv)[4], f4& p) {
+      const _Float16* buf = reinterpret_cast<const _Float16*>(ring + (c % RV) * (64 * H));
 #pragma unroll
-    for (int r = 0; r < 4; r++) vv[r] = *reinterpret_cast<const hv*>(buf + (4 * r + g) * (HD / 4) + i * VD);
-    p = sc[c * 64 + lane];
-  };
-  auto add = [&](int c, const hv (&vv)[4], const f4& p) {
-    float vf[4][VD];
-#pragma unroll
-    for (int r = 0; r < 4; r++)
-#pragma unroll
-      for (int d = 0; d < VD; d++) vf[r][d] = (float)vv[r][d];
-    if (!whole(c)) {
+      for (int r = 0; r < 4; r++) vv[r] = *reinterpret_cast<const hv*>(buf + (4 * r + g) * (HD / 4) + i * VD);
+      p = sc[c * 64 + lane];
+    };
+    auto add = [&](int c, const hv (&vv)[4], const f4& p) {
+      float vf[4][VD];
 #pragma unroll
       for (int r = 0; r < 4; r++)
 #pragma unroll
-        for (int d = 0; d < VD; d++)
-          if (!__builtin_isfinite(vf[r][d])) {
-            vf[r][d] = 0.0f;
-            special = true;
-          }
-    }
+        for (int d = 0; d < VD; d++) vf[r][d] = (float)vv[r][d];
+      if (!whole(c)) {
 #pragma unroll
-    for (int r = 0; r < 4; r++) l = l + p[r];
-    __builtin_amdgcn_sched_barrier(0);
+        for (int r = 0; r < 4; r++)
 #pragma unroll
-    for (int r = 0; r < 4; r++)
-#pragma unroll
-      for (int d = 0; d < VD; d++) o[d] = __builtin_amdgcn_mfma_f32_16x16x1f32(p[r], vf[r][d], o[d], 0, 0, 0);
-  };
-  for (int c = 0; c < nch; c += 2) {  // chunks in pairs: one wait and one LDS round trip for both
-    wait_vm(min(RV - 2, max(0, nch - 2 - c)) * H);  // chunks c and c + 1 have landed
-    __asm__ __volatile__("" ::: "memory");
-    const bool two = c + 1 < nch;
-    hv v0[4], v1[4];
-    f4 p0, p1;
-    load(c, v0, p0);
-    load(two ? c + 1 : c, v1, p1);
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // the slots are free
-    __asm__ __volatile__("" ::: "memory");
-    if (c + RV < nch) issue_v(c + RV);
-    if (c + RV + 1 < nch) issue_v(c + RV + 1);
-    add(c, v0, p0);
-    if (two) add(c + 1, v1, p1);
-  }
-  const bool specials = __builtin_amdgcn_ballot_w64(special) != 0;
-  // record index of the lane's pair, -1 where its row has no item here
-  int rec = -1;
-  if (a < e) rec = (tab[3 * batch + row] + kvh * tab[2 * batch + row] + (s - tab[batch + row])) * G + head;
-  // lane (g, i) holds dims wave*HD/4 + VD*i + (0..VD-1) of pairs 4g..4g+3
-  typedef float fv __attribute__((ext_vector_type(VD)));
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const int pair = 4 * g + k, rk = __shfl(rec, pair, 64);
-    const int pa = __shfl(a, pair, 64), pe = __shfl(e, pair, 64);
-    if (rk < 0) continue;
-    fv x;
-#pragma unroll
-    for (int d = 0; d < VD; d++) x[d] = (o[d][k] + o[d][4 + k]) + (o[d][8 + k] + o[d][12 + k]);
-    if (specials) {
-      // the pair's sums over its non-finite V: an infinity or NaN that any
-      // order of the finite terms leaves as it is
-      for (int t = pa; t < pe; t++) {
-        const int c = (t - T0) >> 4, r = ((t - T0) & 15) >> 2;
-        if (whole(c)) continue;  // chunks that every row sees kept theirs
-        const float p = sc[c * 64 + 16 * (t & 3) + pair][r];
-        const int page = page_table[(size_t)r0 * pps + (t >> ps_shift)];
-        const hv v = *reinterpret_cast<const hv*>(vp + ((size_t)page * page_size + (t & (page_size - 1))) * kvr +
-                                                  kvh * HD + wave * (HD / 4) + i * VD);
-#pragma unroll
-        for (int d = 0; d < VD; d++)
-          if (!__builtin_isfinite((float)v[d])) x[d] += p * (float)v[d];
+          for (int d = 0; d < VD; d++)
+            if (!__builtin_isfinite(vf[r][d])) {
+              vf[r][d] = 0.0f;
+              special = true;
+            }
       }
+#pragma unroll
+      for (int r = 0; r < 4; r++) l = l + p[r];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+#pragma unroll
+        for (int d = 0; d < VD; d++) o[d] = __builtin_amdgcn_mfma_f32_16x16x1f32(p[r], vf[r][d], o[d], 0, 0, 0);
+    };
+    for (int c = 0; c < nch; c += 2) {  // chunks in pairs: one wait and one LDS round trip for both
+      wait_vm(min(RV - 2, max(0, nch - 2 - c)) * H);  // chunks c and c + 1 have landed
+      __asm__ __volatile__("" ::: "memory");
+      const bool two = c + 1 < nch;
+      hv v0[4], v1[4];
+      f4 p0, p1;
+      load(c, v0, p0);
+      load(two ? c + 1 : c, v1, p1);
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // the slots are free
+      __asm__ __volatile__("" ::: "memory");
+      if (c + RV < nch) issue_v(c + RV);
+      if (c + RV + 1 < nch) issue_v(c + RV + 1);
+      add(c, v0, p0);
+      if (two) add(c + 1, v1, p1);
     }
-    *reinterpret_cast<fv*>(part + (size_t)rk * PF + wave * (HD / 4) + VD * i) = x;
-  }
-  l = xor_add<32>(xor_add<16>(l));
-  if (tid < 16 && rec >= 0) {
-    part[(size_t)rec * PF + HD] = mx;
-    part[(size_t)rec * PF + HD + 1] = l;
+    const bool specials = __builtin_amdgcn_ballot_w64(special) != 0;
+    // record index of the lane's pair, -1 where its row has no item here
+    int rec = -1;
+    if (a < e) rec = (rec0 + s) * G + head;
+    // lane (g, i) holds dims wave*HD/4 + VD*i + (0..VD-1) of pairs 4g..4g+3
+    typedef float fv __attribute__((ext_vector_type(VD)));
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const int pair = 4 * g + k, rk = __shfl(rec, pair, 64);
+      const int pa = __shfl(a, pair, 64), pe = __shfl(e, pair, 64);
+      if (rk < 0) continue;
+      fv x;
+#pragma unroll
+      for (int d = 0; d < VD; d++) x[d] = (o[d][k] + o[d][4 + k]) + (o[d][8 + k] + o[d][12 + k]);
+      if (specials) {
+        // the pair's sums over its non-finite V: an infinity or NaN that any
+        // order of the finite terms leaves as it is
+        for (int t = pa; t < pe; t++) {
+          const int c = (t - T0) >> 4, r = ((t - T0) & 15) >> 2;
+          if (whole(c)) continue;  // chunks that every row sees kept theirs
+          const float p = sc[c * 64 + 16 * (t & 3) + pair][r];
+          const int page = page_table[(size_t)r0 * pps + (t >> ps_shift)];
+          const hv v = *reinterpret_cast<const hv*>(vp + ((size_t)page * page_size + (t & (page_size - 1))) * kvr +
+                                                    kvh * HD + wave * (HD / 4) + i * VD);
+#pragma unroll
+          for (int d = 0; d < VD; d++)
+            if (!__builtin_isfinite((float)v[d])) x[d] += p * (float)v[d];
+        }
+      }
+      *reinterpret_cast<fv*>(part + (size_t)rk * PF + wave * (HD / 4) + VD * i) = x;
+    }
+    l = xor_add<32>(xor_add<16>(l));
+    if (tid < 16 && rec >= 0) {
+      part[(size_t)rec * PF + HD] = mx;
+      part[(size_t)rec * PF + HD + 1] = l;
+    }
+    if (z < first && sb - sa >= Z) __syncthreads();  // red and sc are read before the next split writes them
   }
 }
 
@@ -3549,6 +3584,14 @@ hipError_t launch_attn_split_qkv(hipStream_t st, const AttnGeom& g, const AttnQk
 static size_t attn_tile_lds(const AttnGeom& g) {
   return 32768 + 256 + (size_t)((g.split + 15) / 16 + (g.split % 16 ? 1 : 0)) * 1024;
 }
+// Workgroups of a launch at most.  The grid is fixed in the captured graph, so
+// it follows the decoder's capacity, and a workgroup past a short route costs
+// ~1 ns: with one for every split of the capacity, the first 512-row tile of
+// four Llama-3-8B layers at split 64 took 8.2 ms in a decoder for 128 k tokens
+// (2.9 now).  Fewer leave the end of a long route
+// unbalanced: 512 rows behind 30 k tokens, split 256, 16.57 ms at 4096, 16.08 at
+// 8192, 16.03 here, 16.05 with a workgroup for each of the 120 splits.
+static constexpr int64_t kTileWgs = 16384;
 bool attn_tiles(const AttnGeom& g) {
   return (g.hd == 128 || g.hd == 256) && g.page_size % 16 == 0 && (g.page_size & (g.page_size - 1)) == 0 &&
          g.split <= 1024;
@@ -3566,15 +3609,15 @@ hipError_t launch_attn_tile(hipStream_t st, const AttnGeom& g, const float* q, c
                             const int32_t* lane_tab, float* part) {
   if (!attn_tiles(g)) return hipErrorInvalidValue;
   const int shift = __builtin_ctz((unsigned)g.page_size);
-  const int splits = (int)(((int64_t)g.pps * g.page_size + g.split - 1) / g.split);
-  if (splits > 65535) return hipErrorInvalidValue;
+  const int64_t splits = std::min<int64_t>(((int64_t)g.pps * g.page_size + g.split - 1) / g.split, 65535);
 #define RSTR_AT(HD_, G_, L_)                                                                                     \
   {                                                                                                              \
     if constexpr (HD_ >= 128) {                                                                                  \
-      constexpr int RW = 16 / G_;                                                                                \
-      hipLaunchKernelGGL((k_attn_tile<HD_, G_>)   , dim3(g.n_kv, (g.batch + RW - 1) / RW, splits), dim3(256),    \
-                         attn_tile_lds(g), st, g.batch, g.n_kv, g.page_size, shift, g.pps, g.split, g.window,    \
-                         g.scale, q, kpages, vpages, page_table, lengths, lane_tab, part);                       \
+      const int groups = (g.batch + 16 / G_ - 1) / (16 / G_);                                                    \
+      const int64_t z = std::max<int64_t>(1, std::min<int64_t>(splits, kTileWgs / ((int64_t)g.n_kv * groups)));  \
+      hipLaunchKernelGGL((k_attn_tile<HD_, G_>), dim3(g.n_kv, groups, (unsigned)z), dim3(256), attn_tile_lds(g), \
+                         st, g.batch, g.n_kv, g.page_size, shift, g.pps, g.split, g.scale, q, kpages, vpages,    \
+                         page_table, lengths, lane_tab, part);                                                   \
       return hipGetLastError();                                                                                  \
     }                                                                                                            \
   }

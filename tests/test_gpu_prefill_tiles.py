@@ -8,6 +8,8 @@ inside 16-token chunks, chunks and pages, windows that open inside a split, a
 route start other than 0, and infinities in V that some rows of a wave see and
 others do not.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -32,10 +34,10 @@ CASES = [
 ]
 
 
-def _tile(cfg, rows, before, start, ps, split, poison=None):
+def _tile(cfg, rows, before, start, ps, split, poison=None, pps=None):
     n = before + rows
-    pps = -(-n // ps) + 1
-    pages = pps + 3
+    pages = -(-n // ps) + 4
+    pps = pps or -(-n // ps) + 1
     rng = np.random.default_rng(rows * 1000 + before)
     route = rng.permutation(pages).astype(np.int32)[:-(-n // ps)]
     table = np.full(pps, -1, np.int32)
@@ -91,6 +93,47 @@ def test_tiles_match_the_oracle(hd, n_q, n_kv, split, window, ps, rows, before, 
         assert np.isfinite(rows_out).all()
         for i, (a, b) in enumerate(zip(pages, want)):
             assert np.array_equal(a, b), i
+
+
+# (head dim, q heads, kv heads, split, window, rows, rows before the tile, pages a route may have):
+# 2048 (head dim 256: 1024) workgroups a split and a limit of 16384, so a workgroup takes several of the route's
+# splits, which begin at 0 or at the window; and a capacity of more splits than a launch has grid planes
+@pytest.mark.gpu
+@pytest.mark.parametrize("hd,n_q,n_kv,split,window,rows,before,pps", [
+    (128, 64, 8, 32, 0, 512, 100, None), (256, 32, 4, 8, 300, 512, 40, None), (128, 4, 2, 4, 0, 9, 30, 16400)])
+def test_more_splits_than_the_launch_holds(hd, n_q, n_kv, split, window, rows, before, pps):
+    print("case tile splits", hd, n_q, n_kv, split, window, rows, before, pps, flush=True)
+    out, want = _tile(_cfg(hd, n_q, n_kv, window), rows, before, 0, 16, split, pps=pps)
+    for rows_out, pages in out:
+        assert np.isfinite(rows_out).all()
+        for i, (a, b) in enumerate(zip(pages, want)):
+            assert np.array_equal(a, b), i
+
+
+@pytest.mark.gpu
+def test_a_short_route_takes_as_long_in_a_large_decoder():
+    """Routes of 256 tokens, one decoder for 2 k and one for 128 k of context:
+    with a workgroup for every split of the capacity, the second took several
+    times as long."""
+    print("case tile capacity", flush=True)
+    cfg, ps, rows = _cfg(128, 32, 8, 0), 256, 256
+    best = {}
+    with hip.Session(0) as s:
+        m = hip.Model(s, cfg, seed=SEED)
+        p = hip.Pool(m, ps, 4)
+        at = np.arange(rows, dtype=np.int32)
+        for tokens in (2048, 131072):
+            pf = hip.Prefill(m, p, rows, tokens // ps, tokens, 64)
+            table = np.full(tokens // ps, -1, np.int32)
+            table[0] = 1
+            took = []
+            for _ in range(12):
+                t = time.perf_counter()
+                pf.prefill_range(at, ps + at, at, table, rows, 0)
+                took.append(time.perf_counter() - t)
+            best[tokens] = min(took)
+            pf.close()
+    assert best[131072] < 2 * best[2048], best
 
 
 @pytest.mark.gpu
