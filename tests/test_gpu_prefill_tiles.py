@@ -31,6 +31,9 @@ CASES = [
     (256, 8, 1, 100, 70, 16, 5, 333, 0),
     (128, 4, 1, 1028, 0, 16, 21, 1900, 0),   # more than the kernel holds: the work-list kernel
     (128, 4, 2, 32, 0, 8, 21, 50, 0),       # chunks that cross pages: the work-list kernel
+    (128, 4, 1, 64, 0, 16, 1, 300, 0),      # one row: the work-list kernel
+    (256, 4, 1, 32, 24, 16, 1, 61, 2),
+    (256, 4, 1, 32, 24, 16, 2, 60, 0),
 ]
 
 
