@@ -152,11 +152,12 @@ hipError_t launch_attn_prep(hipStream_t st, const AttnGeom& g, const int32_t* le
 hipError_t launch_attn_lists(hipStream_t st, const AttnGeom* g, int n_geo, const int32_t* lengths,
                              int32_t* lane_tab, size_t tab_stride, int max_items);
 // Attention of a bulk-prefill tile (every row a causal lane of one route, all
-// rows of `page_table` alike): the lane tables without the work list, and the
-// split partials of every item as launch_attn_split writes them.
+// rows of `page_table` alike): the lane tables of up to two geometries in one
+// launch, without the work list, and the split partials of every item as
+// launch_attn_split writes them.
 bool attn_tiles(const AttnGeom& g);  // the geometries it serves
-hipError_t launch_attn_tables(hipStream_t st, const AttnGeom& g, const int32_t* lengths, int32_t* lane_tab,
-                              int max_items);
+hipError_t launch_attn_tables(hipStream_t st, const AttnGeom* g, int n_geo, const int32_t* lengths,
+                              int32_t* lane_tab, size_t tab_stride, int max_items);
 hipError_t launch_attn_tile(hipStream_t st, const AttnGeom& g, const float* q, const uint16_t* kpages,
                             const uint16_t* vpages, const int32_t* page_table, const int32_t* lengths,
                             const int32_t* lane_tab, float* part);

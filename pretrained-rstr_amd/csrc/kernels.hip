@@ -1771,13 +1771,20 @@ __device__ __forceinline__ int32_t block_scan(int32_t v, int32_t* s_w, int32_t& 
   return v + before;
 }
 
+// Tables and work lists of up to two geometries, one workgroup each.
+struct AttnListArgs {
+  int window[2], R[2];
+  int32_t* tab[2];
+  int4* items[2];
+};
 // Per-lane item table.  Item (lane b, kv head h, split k) covers the visible
 // tokens [max(lo, k*split), min(len, (k+1)*split)).  A split is full when it
 // holds `split` tokens; only a lane's first (window start) and last split can
 // be partial.
-__global__ __launch_bounds__(1024) void k_attn_prep(int batch, int split, int window, int n_kv, int R,
-                                                   int max_items, const int32_t* __restrict__ lengths,
-                                                   int32_t* __restrict__ tab) {
+__global__ __launch_bounds__(1024) void k_attn_prep(int batch, int split, int n_kv, int max_items,
+                                                   const int32_t* __restrict__ lengths, AttnListArgs args) {
+  const int window = args.window[blockIdx.x], R = args.R[blockIdx.x];
+  int32_t* tab = args.tab[blockIdx.x];
   // tab: lo[B] k0[B] nsplit[B] base[B+1] fbase[B+1] pbase[B+1]; base, fbase
   // and pbase are exclusive prefix sums over lanes of the lane's items, full
   // items and partial items (integer sums: any order is exact)
@@ -1934,11 +1941,6 @@ __global__ __launch_bounds__(256) void k_attn_items(int batch, int n_kv, int spl
 // tables of a step take one launch.  The per-lane and per-item rules are
 // those of the two kernels; the list is the same up to the order inside one
 // partial bucket, which no consumer depends on.
-struct AttnListArgs {
-  int window[2], R[2];
-  int32_t* tab[2];
-  int4* items[2];
-};
 __global__ __launch_bounds__(1024) void k_attn_list(int batch, int split, int n_kv, int max_items,
                                                     const int32_t* __restrict__ lengths, AttnListArgs args) {
   __shared__ int32_t s_w[16], s_h[RSTR_NCH], s_cur[RSTR_NCH];
@@ -2083,8 +2085,11 @@ hipError_t launch_attn_prep(hipStream_t st, const AttnGeom& g, const int32_t* le
   const int R = attn_grid(g, max_items);
   if (R <= 0) return hipErrorInvalidValue;
   if (g.batch >= (1 << 20) || g.n_kv >= (1 << 11)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_attn_prep, dim3(1), dim3(1024), 0, st, g.batch, g.split, g.window, g.n_kv, R,
-                     max_items, lengths, lane_tab);
+  AttnListArgs a{};
+  a.window[0] = g.window;
+  a.R[0] = R;
+  a.tab[0] = lane_tab;
+  hipLaunchKernelGGL(k_attn_prep, dim3(1), dim3(1024), 0, st, g.batch, g.split, g.n_kv, max_items, lengths, a);
   hipLaunchKernelGGL(k_attn_items, dim3((max_items + 255) / 256), dim3(256), 0, st, g.batch, g.n_kv, g.split,
                      lengths, lane_tab, reinterpret_cast<int4*>(lane_tab + attn_items_offset(g.batch)));
   return hipGetLastError();
@@ -3600,10 +3605,18 @@ bool attn_tiles(const AttnGeom& g) {
          g.split <= 1024 && g.batch > 1;
 }
 
-hipError_t launch_attn_tables(hipStream_t st, const AttnGeom& g, const int32_t* lengths, int32_t* lane_tab,
-                              int max_items) {
-  hipLaunchKernelGGL(k_attn_prep, dim3(1), dim3(1024), 0, st, g.batch, g.split, g.window, g.n_kv, 1, max_items,
-                     lengths, lane_tab);
+hipError_t launch_attn_tables(hipStream_t st, const AttnGeom* g, int n_geo, const int32_t* lengths,
+                              int32_t* lane_tab, size_t tab_stride, int max_items) {
+  if (n_geo < 1 || n_geo > 2) return hipErrorInvalidValue;
+  AttnListArgs a{};
+  for (int w = 0; w < n_geo; w++) {
+    if (g[w].batch != g[0].batch || g[w].split != g[0].split || g[w].n_kv != g[0].n_kv) return hipErrorInvalidValue;
+    a.window[w] = g[w].window;
+    a.R[w] = 1;  // no list to claim from
+    a.tab[w] = lane_tab + w * tab_stride;
+  }
+  hipLaunchKernelGGL(k_attn_prep, dim3(n_geo), dim3(1024), 0, st, g[0].batch, g[0].split, g[0].n_kv, max_items, lengths,
+                     a);
   return hipGetLastError();
 }
 

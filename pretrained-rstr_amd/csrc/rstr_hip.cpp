@@ -1375,12 +1375,11 @@ static hipError_t enqueue_step(rstr_decoder* d, hipStream_t st, Prof* prof, bool
   const size_t tabw = d->tabw;
   // a prefill tile's rows share one route: the tile kernel reads the lane tables, not the work list
   const bool tile = !d->head_tail && attn_tiles(geo[0]);
-  if (tile) {
-    for (int w = 0; w < (has_window ? 2 : 1); w++)
-      run(RSTR_K_ROWS, [&] { return launch_attn_tables(st, geo[w], len, d->lane_tab + w * tabw, d->max_items); });
-  } else {
-    run(RSTR_K_ROWS, [&] { return launch_attn_lists(st, geo, has_window ? 2 : 1, len, d->lane_tab, tabw, d->max_items); });
-  }
+  run(RSTR_K_ROWS, [&] {
+    const int n_geo = has_window ? 2 : 1;
+    return tile ? launch_attn_tables(st, geo, n_geo, len, d->lane_tab, tabw, d->max_items)
+                : launch_attn_lists(st, geo, n_geo, len, d->lane_tab, tabw, d->max_items);
+  });
   run(RSTR_K_ROWS, [&] {
     return launch_rms_quant(st, d->r0, d->m->layers[0].attn_norm, goff, md.eps, B, dm, d->act);
   });
