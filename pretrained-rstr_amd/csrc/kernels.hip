@@ -1945,12 +1945,14 @@ __global__ __launch_bounds__(1024) void k_attn_list(int batch, int split, int n_
                                                     const int32_t* __restrict__ lengths, AttnListArgs args) {
   __shared__ int32_t s_w[16], s_h[RSTR_NCH], s_cur[RSTR_NCH];
   __shared__ int32_t s_lo[1024], s_k0[1024], s_ns[1024], s_len[1024], s_base[1025], s_fb[1025];
+  __shared__ int32_t s_long[1024], s_nlong;  // lanes of more than `share` items
   const int gsel = blockIdx.x;
   const int window = args.window[gsel], R = args.R[gsel];
   int32_t* tab = args.tab[gsel];
   int4* items = args.items[gsel];
   const int tid = threadIdx.x;
   for (int i = tid; i < RSTR_NCH; i += 1024) s_h[i] = 0;
+  if (tid == 0) s_nlong = 0;
   __syncthreads();
   // ---- lane tables (k_attn_prep, one chunk of lanes)
   const int b = tid;
@@ -1994,6 +1996,8 @@ __global__ __launch_bounds__(1024) void k_attn_list(int batch, int split, int n_
     tab[4 * batch + 1 + b] = fb_b;
     tab[5 * batch + 2 + b] = pb_b;
   }
+  const int share = max(512, tot_a >> 4);
+  if (n * n_kv > share) s_long[atomicAdd(&s_nlong, 1)] = b;
   s_lo[tid] = l0;
   s_k0[tid] = kk0;
   s_ns[tid] = n;
@@ -2023,17 +2027,16 @@ __global__ __launch_bounds__(1024) void k_attn_list(int batch, int split, int n_
   const int32_t ih = block_scan(hv, s_w, tot_h);
   if (tid < RSTR_NCH) s_cur[RSTR_NCH - 1 - tid] = ih - hv;
   __syncthreads();
-  // ---- the work list (k_attn_items), one wave per lane of the batch: its
-  // items' numbers follow from the lane alone (a search for the lane of every
-  // item cost ~1 us a thousand items)
-  const int wl = tid & 63;
-  for (int bl = __builtin_amdgcn_readfirstlane(tid >> 6); bl < batch; bl += 16) {
-    const int ns = s_ns[bl], n_it = ns * n_kv;
-    if (n_it == 0) continue;
+  // ---- the work list (k_attn_items): an item's entry follows from its lane
+  // and its number there (a search for the lane of every item cost ~1 us a
+  // thousand items)
+  auto entries = [&](int bl, int rel0, int step, int end) {
+    const int ns = s_ns[bl], n_it = min(ns * n_kv, end);
+    if (rel0 >= n_it) return;
     const int ln = s_len[bl], lb = s_lo[bl], k0 = s_k0[bl], ib = s_base[bl], fb = s_fb[bl];
     const int nf = (s_fb[bl + 1] - fb) / n_kv;
     const bool first_partial = !(lb == k0 * split && min(ln, (k0 + 1) * split) - lb == split);
-    for (int rel = wl; rel < n_it; rel += 64) {
+    for (int rel = rel0; rel < n_it; rel += step) {
       const int kvh = rel / ns;
       const int sp = rel - kvh * ns;
       const int k = k0 + sp;
@@ -2048,7 +2051,18 @@ __global__ __launch_bounds__(1024) void k_attn_list(int batch, int split, int n_
       }
       items[pos] = int4{bl | (kvh << 20), t0, t1, ib + rel};
     }
-  }
+  };
+  // One wave writes a lane's first `share` items, all waves together the rest of
+  // a lane that has more, where share is what the waves would have with all items
+  // spread evenly (with a lane to a wave alone, one of 16 k items took 256 passes
+  // of it while the others idled).  Measured on MI355X, us a launch with a lane to
+  // a wave, so shared, and with a search for every item: one lane of 128 k tokens
+  // (split 64, 8 kv heads) 40.3, 12.0 and 18.4; with 19 short lanes 39.8, 12.5, 23.1;
+  // sixteen of 32 k 25.3, 24.8, 64.7.
+  const int wl = tid & 63;
+  for (int bl = __builtin_amdgcn_readfirstlane(tid >> 6); bl < batch; bl += 16) entries(bl, wl, 64, share);
+  const int n_long = s_nlong;
+  for (int i = 0; i < n_long; i++) entries(s_long[i], share + tid, 1024, INT_MAX);
 }
 
 // The step's work lists of up to two geometries (windowed and global layers)

@@ -250,6 +250,15 @@ def test_attention_long_lists_match_oracle(sess, lo, hi):
         m.close()
 
 
+@pytest.mark.parametrize("n_kv,window,B", [(4, 0, 3), (8, 0, 3), (4, 1030, 6), (8, 1030, 40)])
+def test_attention_lists_of_long_lanes_match_oracle(sess, n_kv, window, B):
+    """Lanes of 300 to 2200 items (split 4) beside short and empty ones: the
+    first 512 items of a lane (or a sixteenth of all) are written by its wave,
+    the rest by the whole workgroup, in one pass or two."""
+    print(f"case attention lists of long lanes kv{n_kv} window{window} B{B}", flush=True)
+    _many_splits_case(sess, 64, 2 * n_kv, n_kv, 4, window, B)
+
+
 @pytest.mark.parametrize("window", [0, 40])
 def test_attention_over_1024_lanes_matches_oracle(sess, window):
     """1100 lanes: past the one-workgroup list kernel's 1024 lanes, so the work
