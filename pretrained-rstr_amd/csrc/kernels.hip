@@ -1112,11 +1112,15 @@ __global__ __launch_bounds__(256, 2) void k_qgemm_res(const uint32_t* __restrict
 namespace {
 // The launches k_qgemm_res takes: 2..16 rows, four K slices of at least 14
 // whole chunks (shorter chains are preloaded by k_qgemm), at most one workgroup
-// per CU of a 256-CU device, fragments that fit the LDS.
+// per CU of a 256-CU device, fragments that fit the LDS.  Two rows of a
+// projection under 2048 columns stay with the activation in the launch
+// (launch_qgemm_actin): its few workgroups rebuild little of it, and four layers
+// of 1024 x 7168 took 191 us there against 207 (Q8; Q4 175 and 174), 2048 x 8192
+// 222 and 221, 3072 x 8192 260 and 248.
 bool qgemm_res_serves(const QTensor& w, int mpad, int m_rows, int splits) {
   const int nb = w.k / 32, nchunk = nb / 16;
-  return mpad == 16 && m_rows >= 2 && splits == 4 && nb % 16 == 0 && nchunk >= 14 && nchunk % 2 == 0 &&
-         (w.n / 16 + 3) / 4 * 4 <= 256 && nb / 4 * 1024 <= 160 * 1024;
+  return mpad == 16 && (m_rows > 2 || (m_rows == 2 && w.n >= 2048)) && splits == 4 && nb % 16 == 0 &&
+         nchunk >= 14 && nchunk % 2 == 0 && (w.n / 16 + 3) / 4 * 4 <= 256 && nb / 4 * 1024 <= 160 * 1024;
 }
 hipError_t launch_qgemm_res(hipStream_t st, const QTensor& w, const ActBuf& x, int m_rows, float* y, int ldy,
                             size_t slice_stride) {

@@ -41,14 +41,9 @@ def test_few_rows_over_a_long_k(bits, k, n):
     om.close()
 
 
-# rows, vocabulary: one row is the GEMV; three rows of d_model 256 are 128-column
-# workgroups (256 of them from 32768 up), 64 rows of d_model 512 are 64-column ones
-@pytest.mark.gpu
-@pytest.mark.parametrize("lanes,d,vocab", [(1, 512, 48), (2, 256, 16), (3, 256, 32752), (3, 256, 32768), (2, 512, 1040),
-                                           (64, 512, 16368), (64, 512, 16384), (130, 256, 528)])
-def test_head_slices(lanes, d, vocab):
-    print("case head", lanes, d, vocab, flush=True)
-    cfg = _cfg(4, d_model=d, d_ff=128, vocab=vocab)
+def _step_matches(cfg, lanes):
+    """Two decode steps of one token over one-token routes: tokens, logits and the next rows."""
+    vocab = cfg["vocab"]
     ps, pages, pps, maxpos, split = 16, lanes + 2, 1, 16, 16
     rng = np.random.default_rng(vocab)
     table = rng.permutation(pages).astype(np.int32)[:lanes].reshape(lanes, 1)
@@ -73,3 +68,22 @@ def test_head_slices(lanes, d, vocab):
             assert np.array_equal(dec.rows().view(np.uint32), od.r0().view(np.uint32))
     od.close()
     om.close()
+
+
+# two rows over K = 7168: under 2048 columns the down projection computes its own activation
+@pytest.mark.gpu
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("d", [256, 2048])
+def test_two_lanes_over_a_long_down_projection(bits, d):
+    print("case two lanes", bits, d, flush=True)
+    _step_matches(_cfg(bits, d_model=d, d_ff=7168, vocab=512), 2)
+
+
+# rows, vocabulary: one row is the GEMV; three rows of d_model 256 are 128-column
+# workgroups (256 of them from 32768 up), 64 rows of d_model 512 are 64-column ones
+@pytest.mark.gpu
+@pytest.mark.parametrize("lanes,d,vocab", [(1, 512, 48), (2, 256, 16), (3, 256, 32752), (3, 256, 32768), (2, 512, 1040),
+                                           (64, 512, 16368), (64, 512, 16384), (130, 256, 528)])
+def test_head_slices(lanes, d, vocab):
+    print("case head", lanes, d, vocab, flush=True)
+    _step_matches(_cfg(4, d_model=d, d_ff=128, vocab=vocab), lanes)
