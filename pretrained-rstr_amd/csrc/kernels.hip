@@ -1190,16 +1190,26 @@ int qgemm_splits(int n, int mpad, int bits) {
 }
 
 // K slices of the LM head: one, unless that leaves CUs without a workgroup
-// (small vocabularies), where the tail adds four slices as it reads them.
-// Measured on MI355X, 4096 x 4096 Q4: 35.7 us in one slice at 16 rows (16
-// workgroups), 28.4 at 45, 27.6 at 128 (128 workgroups).  One row (and two over
-// K <= 1024) takes the GEMV, one workgroup per column tile.
+// (vocabularies smaller than any full model's here), where the tail adds four
+// slices as it reads them.  Measured on MI355X, 4096 x 4096 Q4: 35.7 us in one
+// slice at 16 rows (16 workgroups), 28.4 at 45, 27.6 at 128 (128 workgroups).
+// Slices shorten a wave's chain, which is as long as K and the row tiles of its
+// workgroup, and move the logits five times instead of once, so a short chain
+// pays at fewer logits.  Steps of one layer, us at one slice and at four:
+//   K = 4096: 3 x 50256 131 and 116, 64 x 16128 161 and 154, 128 x 16128 222 and 223
+//   K = 1024: 3 x 50256 70.1 and 66.7, 64 x 8192 80.6 and 77.3, 16 x 50256 73.3
+//     and 74.7, 32 x 32000 79.1 and 83.4
+//   K = 640: 45 x 8192 72.2 and 70.7, 1 x 16384 (128 workgroups) 57.7 and 56.2,
+//     1 x 32000 (250) 58.5 and 59.8, 32 x 16128 72.7 and 73.7, 64 x 16128 74.6
+//     and 77.8; four layers 128 x 4096 216 and 208
+// One row (and two over K <= 1024) takes the GEMV, one workgroup per column tile.
 int qgemm_head_splits(int n, int k, int rows, int bits) {
   const int nb = k / 32, mt_all = (rows + 15) / 16;
   if ((nb / 4) % 4 == 0 && (rows == 1 || (rows == 2 && k <= 1024))) return 1;
   const QgPlan p = qg_plan(16 * mt_all, 1, bits, nb);
   const int per = 4 * p.ct;
-  return (n / 16 + per - 1) / per * ((mt_all + p.rt - 1) / p.rt) < 256 ? 4 : 1;
+  const int wgs = (n / 16 + per - 1) / per * ((mt_all + p.rt - 1) / p.rt);
+  return wgs < (k >= 1024 ? 256 : 192) && (int64_t)rows * n <= 256 * ((int64_t)k * std::max(p.rt, 2) / 2 + 1024) ? 4 : 1;
 }
 
 // Launch arguments of one projection and the chunking choices made for it.

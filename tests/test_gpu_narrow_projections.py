@@ -80,10 +80,14 @@ def test_two_lanes_over_a_long_down_projection(bits, d):
 
 
 # rows, vocabulary: one row is the GEMV; three rows of d_model 256 are 128-column
-# workgroups (256 of them from 32768 up), 64 rows of d_model 512 are 64-column ones
+# workgroups (four slices up to 191 of them), of d_model 1024 256-column ones (255);
+# 64 rows of d_model 512 stay at one slice from 524 288 logits on, of 2048 from 256
+# 64-column workgroups on
 @pytest.mark.gpu
-@pytest.mark.parametrize("lanes,d,vocab", [(1, 512, 48), (2, 256, 16), (3, 256, 32752), (3, 256, 32768), (2, 512, 1040),
-                                           (64, 512, 16368), (64, 512, 16384), (130, 256, 528)])
+@pytest.mark.parametrize("lanes,d,vocab", [(1, 512, 48), (2, 256, 16), (3, 256, 24448), (3, 256, 24464), (3, 256, 32768),
+                                           (3, 1024, 65280), (3, 1024, 65296), (2, 512, 1040), (64, 512, 8192),
+                                           (64, 512, 8208), (64, 512, 16384), (64, 2048, 16320), (64, 2048, 16336),
+                                           (130, 256, 528)])
 def test_head_slices(lanes, d, vocab):
     print("case head", lanes, d, vocab, flush=True)
     _step_matches(_cfg(4, d_model=d, d_ff=128, vocab=vocab), lanes)
