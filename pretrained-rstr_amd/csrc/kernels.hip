@@ -2764,12 +2764,12 @@ __device__ __forceinline__ float qk_tree(float (&v)[G], int j) {
 // 99), because a workgroup here has nothing in flight while it computes.
 // Every list position is static here, so no claims.
 //
-// QKV: the item's query comes from the qkv projection slices through
-// attn_qkv_prologue (q is unused); the lane's newest K/V row is appended by the
-// item that holds it, which takes the row from LDS, not from the page.
+// QKV: the item's query comes from the qkv projection slices (QkvHeads; q is
+// unused); the lane's newest K/V row is appended by the item that holds it, which
+// takes the row from LDS, not from the page.
 template <int HD, int G, int NC, bool QKV = false, bool DIRECT = false>
 __global__ __launch_bounds__(256, QKV ? (NC == 4 && G <= 4 && HD == 128 ? 3 : 1)
-                                      : (NC == 4 && G <= 4 && HD == 128 ? 4 : 2)) void k_attn_item(
+                                      : (HD == 128 && G <= 4 ? (NC == 4 ? 4 : 3) : 2)) void k_attn_item(
     int n_kv, int page_size, int ps_shift, int pps, float scale,
     const float* __restrict__ q, const uint16_t* kp, const uint16_t* vp,
     const int32_t* __restrict__ page_table, const int32_t* __restrict__ n_items,
@@ -3454,11 +3454,21 @@ struct AttnSplit {
   }
   static int ring(const AttnGeom& g) { return waves_per_cu(g, RBS) > waves_per_cu(g, RB) ? RBS : RB; }
   // Few-item launches (k_attn_item, one 4-wave workgroup per item): head dim
-  // 128 or 256, whole-page chunks, and a largest work list that fits in two
+  // 128 or 256, whole-page chunks, and a largest work list that fits in kRounds
   // rounds of resident workgroups.  Its segments hold 64 tokens for splits up
-  // to 64, else 256 (head dim 256: 128), as far as a thread's registers go.
+  // to 64 and for groups of 8, else 128: with 256 (head dim 128) two workgroups
+  // fit a CU instead of three, and half the list sizes that the kernel is the
+  // better one for went to the one-wave kernel.  Steps of four layers, us with
+  // segments of 256 and of 128: 48 Qwen3-0.6B lanes of 2 k, split 1024, 519 and
+  // 359; 32 lanes of 300 tokens, split 128, 255 and 228; 8 lanes of 300 tokens in
+  // a decoder for 4 k, split 256, 230 and 176.
   static constexpr bool kWG = HD == 128 || HD == 256;
-  static constexpr int NCB = G == 8 ? 4 : HD == 128 ? 16 : 8;
+  static constexpr int NCB = G == 8 ? 4 : 8;
+  // At head dim 256 the one-wave kernel holds few waves a CU and stays behind
+  // to far longer lists: 64 Gemma-3-270M lanes of 4 k, split 256 (1152 items),
+  // 362 us there and 234 here, 128 lanes (2304) 404 and 284, at split 64 (8448)
+  // 286 and 273; with groups of 1 and 2 they draw even from 1100 items on.
+  static constexpr int kRounds = HD == 256 ? (G >= 4 ? 16 : 4) : 2;
   template <bool QKV, bool DIRECT>
   static decltype(&k_attn_item<HD, G, 4, QKV, DIRECT>) item_kernel(const AttnGeom& g) {
     return g.split > 64 ? k_attn_item<HD, G, NCB, QKV, DIRECT> : k_attn_item<HD, G, 4, QKV, DIRECT>;
@@ -3486,7 +3496,7 @@ struct AttnSplit {
   static bool use_wg(const AttnGeom& g, int max_items) {
     if (!kWG || !pg16(g)) return false;
     const int cap = wg_capacity<QKV>(g);
-    return cap > 0 && max_items <= (QKV ? 1 : 2) * cap;
+    return cap > 0 && max_items <= (QKV ? 1 : kRounds) * cap;
   }
   static int grid(const AttnGeom& g, int max_items) {
     if (use_wg(g, max_items)) return std::max(1, std::min(wg_capacity(g), max_items));

@@ -250,6 +250,17 @@ def test_attention_long_lists_match_oracle(sess, lo, hi):
         m.close()
 
 
+@pytest.mark.parametrize("hd,n_q,n_kv,split,window,B", [
+    (256, 8, 2, 16, 0, 60), (256, 4, 4, 16, 0, 12), (128, 8, 2, 128, 0, 9), (128, 8, 2, 132, 0, 9),
+    (128, 4, 4, 264, 300, 7), (128, 16, 2, 132, 0, 6), (256, 4, 1, 136, 40, 7)])
+def test_attention_few_item_segments_match_oracle(sess, hd, n_q, n_kv, split, window, B):
+    """The few-item kernel over several rounds of resident workgroups (head dim
+    256) and over splits of one 128-token segment, a segment and a chunk, and
+    three segments, with partial last ones and windows."""
+    print(f"case attention segments hd{hd} q{n_q} kv{n_kv} split{split} window{window} B{B}", flush=True)
+    _many_splits_case(sess, hd, n_q, n_kv, split, window, B)
+
+
 @pytest.mark.parametrize("n_kv,window,B", [(4, 0, 3), (8, 0, 3), (4, 1030, 6), (8, 1030, 40)])
 def test_attention_lists_of_long_lanes_match_oracle(sess, n_kv, window, B):
     """Lanes of 300 to 2200 items (split 4) beside short and empty ones: the
