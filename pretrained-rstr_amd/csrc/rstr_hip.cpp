@@ -54,11 +54,32 @@ int fail(rstr_session* s, int code, const std::string& msg) {
                   std::string(#expr) + ": " + hipGetErrorString(e_));                    \
   } while (0)
 
+// Device and pinned memory.  An allocation that does not fit is tried again
+// without the blocks that the pools of this GPU keep for isolated attention.
+bool release_kept_blocks();
+template <class T>
+hipError_t dev_alloc(T** p, size_t bytes) {
+  *p = nullptr;
+  hipError_t e = hipMalloc((void**)p, bytes);
+  if (e == hipErrorOutOfMemory && release_kept_blocks()) {
+    (void)hipGetLastError();  // the first attempt's error
+    e = hipMalloc((void**)p, bytes);
+  }
+  return e;
+}
+template <class T>
+hipError_t host_alloc(T** p, size_t bytes) {
+  *p = nullptr;
+  hipError_t e = hipHostMalloc((void**)p, bytes);
+  if (e == hipErrorOutOfMemory && release_kept_blocks()) {
+    (void)hipGetLastError();
+    e = hipHostMalloc((void**)p, bytes);
+  }
+  return e;
+}
 template <class T>
 hipError_t dmalloc(T** p, size_t elems) {
-  *p = nullptr;
-  if (elems == 0) elems = 1;
-  return hipMalloc((void**)p, elems * sizeof(T));
+  return dev_alloc(p, std::max<size_t>(elems, 1) * sizeof(T));
 }
 
 inline int64_t linear_bytes(int bits, int n, int k) { return (int64_t)n * k / 32 * (bits == 4 ? 16 : 32); }
@@ -111,7 +132,7 @@ struct HostRing {
       if (h[k]) hipHostFree(h[k]);
       h[k] = nullptr;
       cap[k] = 0;
-      if ((e = hipHostMalloc((void**)&h[k], sizeof(int32_t) * std::max<size_t>(na + nb, 64))) != hipSuccess) return e;
+      if ((e = host_alloc(&h[k], sizeof(int32_t) * std::max<size_t>(na + nb, 64))) != hipSuccess) return e;
       cap[k] = std::max<size_t>(na + nb, 64);
     }
     if (na) std::memcpy(h[k], a, sizeof(int32_t) * na);
@@ -161,11 +182,35 @@ struct rstr_pool {
   void* attn_dev = nullptr;
   void* attn_host = nullptr;
   size_t attn_dev_bytes = 0, attn_host_bytes = 0;
-  std::mutex attn_mu;  // held by the call that uses them
+  bool attn_busy = false;  // a call uses them
 };
 // What a pool keeps for the isolated attention between calls, per buffer;
 // larger calls, and calls that find the buffers in use, allocate and free their own.
 static constexpr size_t kAttnKeep = (size_t)128 << 20;
+// The open pools; guards the list and every pool's attn_busy and idle blocks.
+static std::mutex g_pools_mu;
+static std::vector<rstr_pool*> g_pools;
+
+static bool free_attn_blocks(rstr_pool* p) {
+  const bool any = p->attn_dev || p->attn_host;
+  if (p->attn_dev) hipFree(p->attn_dev);
+  if (p->attn_host) hipHostFree(p->attn_host);
+  p->attn_dev = p->attn_host = nullptr;
+  p->attn_dev_bytes = p->attn_host_bytes = 0;
+  return any;
+}
+namespace {
+// Frees the idle blocks of the current GPU's pools; false if there were none.
+bool release_kept_blocks() {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  std::lock_guard<std::mutex> lock(g_pools_mu);
+  bool any = false;
+  for (rstr_pool* p : g_pools)
+    if (!p->attn_busy && p->m->s->device == dev) any |= free_attn_blocks(p);
+  return any;
+}
+}  // namespace
 
 struct rstr_transfer {
   rstr_pool* p = nullptr;
@@ -183,7 +228,7 @@ static hipError_t ensure_templates(rstr_pool* p, uint64_t seed) {
   if (p->tmpl_ready && p->tmpl_seed == seed) return hipSuccess;
   int L = p->m->d.n_layers;
   if (!p->tmpl) {
-    hipError_t e = hipMalloc(&p->tmpl, sizeof(uint16_t) * (size_t)2 * L * RSTR_SYNTH_TEMPLATES * p->page_elems);
+    hipError_t e = dev_alloc(&p->tmpl, sizeof(uint16_t) * (size_t)2 * L * RSTR_SYNTH_TEMPLATES * p->page_elems);
     if (e != hipSuccess) return e;
   }
   hipError_t e = launch_gen_templates(p->m->s->stream, p->tmpl, L, p->page_elems, seed);
@@ -344,7 +389,7 @@ static int alloc_q(rstr_model* m, QTensor& t, int n, int k) {
   t.k = k;
   t.bits = m->d.weight_bits;
   int64_t wb = linear_bytes(t.bits, n, k);
-  HIPCHK(m->s, hipMalloc(&t.w, (size_t)wb));
+  HIPCHK(m->s, dev_alloc(&t.w, (size_t)wb));
   m->allocs.push_back(t.w);
   HIPCHK(m->s, dmalloc(&t.s, (size_t)n * (k / 32)));
   m->allocs.push_back(t.s);
@@ -535,7 +580,7 @@ static int bind_tensors(rstr_session* s, const rstr_model_desc* desc, int32_t n_
     if (need > tmp_cap) {
       if (tmp) hipFree(tmp);
       tmp = nullptr;
-      if (hipMalloc(&tmp, need * sizeof(float)) != hipSuccess) return bail(RSTR_E_OOM, "hipMalloc");
+      if (dev_alloc(&tmp, need * sizeof(float)) != hipSuccess) return bail(RSTR_E_OOM, "hipMalloc");
       tmp_cap = need;
     }
     if (t.dtype == 0) {
@@ -545,7 +590,7 @@ static int bind_tensors(rstr_session* s, const rstr_model_desc* desc, int32_t n_
       if (need * esz > raw_cap) {
         if (raw) hipFree(raw);
         raw = nullptr;
-        if (hipMalloc(&raw, need * esz) != hipSuccess) return bail(RSTR_E_OOM, "hipMalloc");
+        if (dev_alloc(&raw, need * esz) != hipSuccess) return bail(RSTR_E_OOM, "hipMalloc");
         raw_cap = need * esz;
       }
       if (hipMemcpy(raw, t.data, need * esz, hipMemcpyHostToDevice) != hipSuccess ||
@@ -689,7 +734,7 @@ extern "C" int rstr_pool_open(rstr_model* m, int32_t page_size, int32_t physical
   };
   for (int i = 0; i < 2 * L; i++) {
     uint16_t* q = nullptr;
-    hipError_t e = hipMalloc(&q, slab_elems * 2);
+    hipError_t e = dev_alloc(&q, slab_elems * 2);
     if (e != hipSuccess) {
       cleanup();
       return fail(s, RSTR_E_OOM, "page pool slab allocation failed");
@@ -701,7 +746,7 @@ extern "C" int rstr_pool_open(rstr_model* m, int32_t page_size, int32_t physical
     }
   }
   if (dmalloc(&p->d_slabs, 2 * L) != hipSuccess || dmalloc(&p->d_pairs, 2) != hipSuccess ||
-      hipHostMalloc((void**)&p->h_pairs, 2 * sizeof(int32_t)) != hipSuccess) {
+      host_alloc(&p->h_pairs, 2 * sizeof(int32_t)) != hipSuccess) {
     cleanup();
     return fail(s, RSTR_E_OOM, "page pool tables");
   }
@@ -711,6 +756,10 @@ extern "C" int rstr_pool_open(rstr_model* m, int32_t page_size, int32_t physical
     cleanup();
     return fail(s, RSTR_E_HIP, "page pool setup");
   }
+  {
+    std::lock_guard<std::mutex> lock(g_pools_mu);
+    g_pools.push_back(p.get());
+  }
   *out = p.release();
   return RSTR_OK;
 }
@@ -719,6 +768,10 @@ extern "C" int rstr_pool_close(rstr_pool* p) {
   if (!p) return RSTR_OK;
   if (p->open_transfers > 0) return fail(p->m->s, RSTR_E_STATE, "pool has chunk transfers in flight");
   hipSetDevice(p->m->s->device);
+  {
+    std::lock_guard<std::mutex> lock(g_pools_mu);
+    g_pools.erase(std::remove(g_pools.begin(), g_pools.end(), p), g_pools.end());
+  }
   hipStreamSynchronize(p->m->s->stream);
   for (auto* q : p->slabs) hipFree(q);
   hipFree(p->d_slabs);
@@ -729,8 +782,7 @@ extern "C" int rstr_pool_close(rstr_pool* p) {
   if (p->tmpl) hipFree(p->tmpl);
   if (p->stage) hipFree(p->stage);
   if (p->d_chunk_pages) hipFree(p->d_chunk_pages);
-  if (p->attn_dev) hipFree(p->attn_dev);
-  if (p->attn_host) hipHostFree(p->attn_host);
+  free_attn_blocks(p);
   for (auto& b : p->pinned) hipHostFree(b.first);
   delete p;
   return RSTR_OK;
@@ -775,7 +827,7 @@ static int chunk_submit(rstr_pool* p, const int32_t* pages, int32_t n_pages, int
       if (p->stage) hipFree(p->stage);
       p->stage = nullptr;
       p->stage_bytes = 0;
-      if (hipMalloc(&p->stage, pbytes) != hipSuccess) return fail(s, RSTR_E_OOM, "chunk staging allocation failed");
+      if (dev_alloc(&p->stage, pbytes) != hipSuccess) return fail(s, RSTR_E_OOM, "chunk staging allocation failed");
       p->stage_bytes = pbytes;
     }
     if (p->chunk_pages_cap < n_pages) {
@@ -803,7 +855,7 @@ static int chunk_submit(rstr_pool* p, const int32_t* pages, int32_t n_pages, int
     t->host_bytes = p->pinned[best].second;
     p->pinned.erase(p->pinned.begin() + best);
   } else {
-    if (hipHostMalloc(&t->host, need) != hipSuccess) return fail(s, RSTR_E_OOM, "pinned chunk buffer allocation failed");
+    if (host_alloc(&t->host, need) != hipSuccess) return fail(s, RSTR_E_OOM, "pinned chunk buffer allocation failed");
     t->host_bytes = need;
   }
   auto cleanup = [&]() {
@@ -1102,13 +1154,13 @@ static int decoder_open(rstr_model* m, rstr_pool* p, int32_t batch, int32_t pps,
   A(dmalloc(&d->amax_cand, (size_t)2 * batch * argmax_segments(batch, md.vocab)));
   A(dmalloc(&d->d_lanes, (size_t)batch));
   A(dmalloc(&d->d_tokens, (size_t)batch));
-  if (e == hipSuccess) e = hipHostMalloc((void**)&d->h_desc, sizeof(int32_t) * d->desc_words);
-  if (e == hipSuccess) e = hipHostMalloc((void**)&d->h_tok, sizeof(int32_t) * batch);
+  if (e == hipSuccess) e = host_alloc(&d->h_desc, sizeof(int32_t) * d->desc_words);
+  if (e == hipSuccess) e = host_alloc(&d->h_tok, sizeof(int32_t) * batch);
   for (hipEvent_t& ev : d->ev_step)
     if (e == hipSuccess) e = hipEventCreate(&ev);
   for (int i = 0; i < 2; i++) {
-    if (e == hipSuccess) e = hipHostMalloc((void**)&d->h_desc_q[i], sizeof(int32_t) * d->desc_words);
-    if (e == hipSuccess) e = hipHostMalloc((void**)&d->h_tok_q[i], sizeof(int32_t) * batch);
+    if (e == hipSuccess) e = host_alloc(&d->h_desc_q[i], sizeof(int32_t) * d->desc_words);
+    if (e == hipSuccess) e = host_alloc(&d->h_tok_q[i], sizeof(int32_t) * batch);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&d->ev_q[i], hipEventDisableTiming);
   }
   if (e != hipSuccess) {
@@ -2095,30 +2147,44 @@ extern "C" int rstr_attention_run(rstr_pool* p, int32_t layer, int32_t batch, in
       if (host) hipHostFree(host);
     }
   } own;
-  std::unique_lock<std::mutex> kept(p->attn_mu, std::try_to_lock);
-  void *dev = kept ? p->attn_dev : nullptr, *host = kept ? p->attn_host : nullptr;
-  if (!kept || bk.total > p->attn_dev_bytes) {
-    if (kept && p->attn_dev) {
+  struct Claim {
+    rstr_pool* p = nullptr;
+    ~Claim() {
+      if (!p) return;
+      std::lock_guard<std::mutex> lock(g_pools_mu);
+      p->attn_busy = false;
+    }
+  } kept;
+  {
+    std::lock_guard<std::mutex> lock(g_pools_mu);
+    if (!p->attn_busy) {
+      p->attn_busy = true;
+      kept.p = p;
+    }
+  }
+  void *dev = kept.p ? p->attn_dev : nullptr, *host = kept.p ? p->attn_host : nullptr;
+  if (!kept.p || bk.total > p->attn_dev_bytes) {
+    if (kept.p && p->attn_dev) {
       hipFree(p->attn_dev);
       p->attn_dev = nullptr;
       p->attn_dev_bytes = 0;
     }
-    HIPCHK(s, hipMalloc(&dev, bk.total));
-    if (kept && bk.total <= kAttnKeep) {
+    HIPCHK(s, dev_alloc(&dev, bk.total));
+    if (kept.p && bk.total <= kAttnKeep) {
       p->attn_dev = dev;
       p->attn_dev_bytes = bk.total;
     } else {
       own.dev = dev;
     }
   }
-  if (!kept || host_bytes > p->attn_host_bytes) {
-    if (kept && p->attn_host) {
+  if (!kept.p || host_bytes > p->attn_host_bytes) {
+    if (kept.p && p->attn_host) {
       hipHostFree(p->attn_host);
       p->attn_host = nullptr;
       p->attn_host_bytes = 0;
     }
-    HIPCHK(s, hipHostMalloc(&host, host_bytes));
-    if (kept && host_bytes <= kAttnKeep) {
+    HIPCHK(s, host_alloc(&host, host_bytes));
+    if (kept.p && host_bytes <= kAttnKeep) {
       p->attn_host = host;
       p->attn_host_bytes = host_bytes;
     } else {
