@@ -1122,6 +1122,12 @@ bool qgemm_res_serves(const QTensor& w, int mpad, int m_rows, int splits) {
   return mpad == 16 && (m_rows > 2 || (m_rows == 2 && w.n >= 2048)) && splits == 4 && nb % 16 == 0 &&
          nchunk >= 14 && nchunk % 2 == 0 && (w.n / 16 + 3) / 4 * 4 <= 256 && nb / 4 * 1024 <= 160 * 1024;
 }
+// D, the chunks in flight, divides the chunk count (no tail).  Steps of four
+// layers at eight rows, us: K = 14336 (28 chunks), Q4 with 7 in flight 271, 4 282,
+// 2 284; Q8, whose chunk is twice the registers, 367, 353, 352; K = 7168 (14), Q4 7
+// and 2 169 and 174, Q8 199 and 189; 16 to 40 chunks 4 and 2 within 1.5%.  Odd
+// counts stay with k_qgemm: no model has one (4096 x 7680 with 3 in flight 236,
+// there 248).
 hipError_t launch_qgemm_res(hipStream_t st, const QTensor& w, const ActBuf& x, int m_rows, float* y, int ldy,
                             size_t slice_stride) {
   const int nb = w.k / 32, nct = w.n / 16, nchunk = nb / 16;
@@ -1130,11 +1136,11 @@ hipError_t launch_qgemm_res(hipStream_t st, const QTensor& w, const ActBuf& x, i
 #define RSTR_RES(B_, D_)                                                                                              \
   hipLaunchKernelGGL((k_qgemm_res<B_, D_>), grid, dim3(256), lds, st, (const uint32_t*)w.w, w.s, x.q, nb, nct, y, ldy, \
                      m_rows, slice_stride)
-#define RSTR_RES_D(B_)                            \
-  do {                                            \
-    if (nchunk % 7 == 0) RSTR_RES(B_, 7);         \
-    else if (nchunk % 4 == 0) RSTR_RES(B_, 4);    \
-    else RSTR_RES(B_, 2);                         \
+#define RSTR_RES_D(B_)                              \
+  do {                                              \
+    if (B_ == 4 && nchunk % 7 == 0) RSTR_RES(4, 7); \
+    else if (nchunk % 4 == 0) RSTR_RES(B_, 4);      \
+    else RSTR_RES(B_, 2);                           \
   } while (0)
   if (w.bits == 4) RSTR_RES_D(4);
   else RSTR_RES_D(8);
