@@ -1,9 +1,10 @@
 """Projections whose launches leave CUs idle, against the oracle bit for bit.
 
 - Two to sixteen rows against a long K (weights streamed past resident
-  activations): the smallest K it takes and every chunk-group width it has,
-  column tiles that do and do not fill a workgroup, row counts at both ends, and
-  the shapes next to its limits, which other forms serve.
+  activations): the smallest K it takes and every chunk-group width it has, the
+  largest K (20480: 160 KB of LDS) and width (4096 columns), column tiles that do
+  and do not fill a workgroup, row counts at both ends, and the shapes next to
+  its limits, which other forms serve.
 - The LM head in four K slices that the tail adds: vocabularies on both sides of
   the line, where the next token's row and the logits read back come from the
   added slices.
@@ -23,8 +24,8 @@ def _cfg(bits, **kw):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("bits", [4, 8])
-@pytest.mark.parametrize("k,n", [(7168, 256), (8192, 128), (9216, 384), (6656, 128), (40960, 128), (41472, 128),
-                                 (7168, 4224)])
+@pytest.mark.parametrize("k,n", [(7168, 256), (8192, 128), (9216, 384), (6656, 128), (14336, 128),
+                                 (20480, 128), (21504, 128), (7168, 4096), (7168, 4224)])
 def test_few_rows_over_a_long_k(bits, k, n):
     print("case long k", bits, k, n, flush=True)
     cfg = _cfg(bits, d_model=n, d_ff=k, vocab=512)
