@@ -1,9 +1,11 @@
 """Bulk-prefill tiles through the matrix-instruction attention kernel (head dims
 128 and 256) against the oracle, which runs the tile's rows as causal lanes with
-the decode step's reduction order: final rows and every layer's K/V bit for bit.
+the decode step's reduction order: every layer's K/V bit for bit, and the final
+rows, whose logits through the oracle's own final norm and head have to be the
+bits of the logits that its step reports.
 
 Sizes are where the kernel can go wrong: row groups of every GQA width (16/G
-rows per wave, 64/G per workgroup) with a remainder, splits that start and end
+rows per workgroup) with a remainder, splits that start and end
 inside 16-token chunks, chunks and pages, windows that open inside a split, a
 route start other than 0, and infinities in V that some rows of a wave see and
 others do not.
@@ -77,6 +79,12 @@ def _tile(cfg, rows, before, start, ps, split, poison=None, pps=None):
             out.append((pf.rows_out(), [p.pages(k, layer).view(np.uint16).ravel() for layer in range(cfg["n_layers"])
                                         for k in (0, 1)]))
     want = [od.slab(k, layer).view(np.uint16).ravel().copy() for layer in range(cfg["n_layers"]) for k in (0, 1)]
+    if poison is None:
+        want.append(od.logits().view(np.uint32))
+        for rows_out, pages in out:
+            assert np.isfinite(rows_out).all()
+            h = O.rmsnorm(rows_out, om.norm(-1, "final_norm"), float(cfg["gain_offset"]), cfg["eps"])
+            pages.append(O.qlinear(cfg["weight_bits"], *om.tensor(-1, "embed"), *O.quant_act(h)).view(np.uint32))
     od.close()
     om.close()
     return out, want
@@ -92,9 +100,8 @@ def _cfg(hd, n_q, n_kv, window):
 def test_tiles_match_the_oracle(hd, n_q, n_kv, split, window, ps, rows, before, start):
     print("case tile", hd, n_q, n_kv, split, window, ps, rows, before, start, flush=True)
     out, want = _tile(_cfg(hd, n_q, n_kv, window), rows, before, start, ps, split)
-    for rows_out, pages in out:
-        assert np.isfinite(rows_out).all()
-        for i, (a, b) in enumerate(zip(pages, want)):
+    for _, pages in out:
+        for i, (a, b) in enumerate(zip(pages, want, strict=True)):
             assert np.array_equal(a, b), i
 
 
@@ -107,9 +114,8 @@ def test_tiles_match_the_oracle(hd, n_q, n_kv, split, window, ps, rows, before, 
 def test_more_splits_than_the_launch_holds(hd, n_q, n_kv, split, window, rows, before, pps):
     print("case tile splits", hd, n_q, n_kv, split, window, rows, before, pps, flush=True)
     out, want = _tile(_cfg(hd, n_q, n_kv, window), rows, before, 0, 16, split, pps=pps)
-    for rows_out, pages in out:
-        assert np.isfinite(rows_out).all()
-        for i, (a, b) in enumerate(zip(pages, want)):
+    for _, pages in out:
+        for i, (a, b) in enumerate(zip(pages, want, strict=True)):
             assert np.array_equal(a, b), i
 
 
@@ -140,7 +146,7 @@ def test_a_short_route_takes_as_long_in_a_large_decoder():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("hd,window", [(128, 0), (256, 24)])
+@pytest.mark.parametrize("hd,window", [(128, 0), (128, 24), (256, 24)])
 def test_infinite_values_reach_only_the_rows_that_see_them(hd, window):
     """V = inf (and NaN) at cached tokens: with a window, rows of one wave see
     them or not, and the K/V each row appends follows the oracle's."""
@@ -159,11 +165,11 @@ def test_infinite_values_reach_only_the_rows_that_see_them(hd, window):
 @pytest.mark.parametrize("d_model,d_ff,n_q,n_kv", [(640, 256, 16, 8), (4096, 512, 4, 2)])
 def test_large_tiles_in_two_slices_match_the_oracle(d_model, d_ff, n_q, n_kv, bits):
     """At 449 rows a 4096-wide projection runs in two K slices: the qkv
-    projection over K = 640 (quarters of five blocks), or o and down."""
+    projection over K = 640 (quarters of five blocks), or o and down (the last
+    layer's through the logits)."""
     print("case two slices", d_model, bits, flush=True)
     cfg = dict(_cfg(128, n_q, n_kv, 0), n_layers=2, d_model=d_model, d_ff=d_ff, weight_bits=bits)
     out, want = _tile(cfg, 449, 20, 0, 16, 256)
-    for rows_out, pages in out:
-        assert np.isfinite(rows_out).all()
-        for i, (a, b) in enumerate(zip(pages, want)):
+    for _, pages in out:
+        for i, (a, b) in enumerate(zip(pages, want, strict=True)):
             assert np.array_equal(a, b), i
