@@ -527,6 +527,11 @@ def class_rates(cfg: dict, prof: dict, n_steps: int, prof_plan: list, weight_byt
     return out
 
 
+def profiler_loaded(environ) -> bool:
+    """Whether rocprofv3 runs this process (it names its tool library in the environment)."""
+    return "ROCP_TOOL_LIBRARIES" in environ or any(k.startswith("ROCPROF_") for k in environ)
+
+
 def live_loop(args, cfg, lanes, ps, physical, maxpos, prompt, output, arrivals, seed, dec, pool) -> dict:
     """The serving loop in the sense of continuation/benchmark.clj:180-194: every
     step is planned by the host control plane and run through one
@@ -628,6 +633,11 @@ def main():
     args = ap.parse_args()
     if args.split is None:
         args.split = SPLITS[args.workload]
+    if args.live_steps > 0 and profiler_loaded(os.environ):
+        # a traced live loop has ended the process with a malformed queue packet
+        # (the runtime's report; the same loop untraced runs): not run under a profiler
+        log("a profiler is loaded: the live loop is skipped")
+        args.live_steps = 0
     if args.gpus != 1:
         print(json.dumps({"error": "this build measures one GPU; --gpus must be 1 (the decode step "
                                    "shards as independent per-GPU replicas with their own lanes and "
