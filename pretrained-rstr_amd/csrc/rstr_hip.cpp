@@ -1982,18 +1982,9 @@ extern "C" int rstr_linear_run(rstr_model* m, int32_t layer, int32_t role, int32
 // ---------------------------------------------------------------------------
 // isolated routed attention
 // ---------------------------------------------------------------------------
-struct AttnBufs {
-  float *q = nullptr, *out = nullptr, *part = nullptr;
-  int32_t *pt = nullptr, *len = nullptr, *tab = nullptr;
-  ~AttnBufs() {
-    for (void* p : {(void*)q, (void*)out, (void*)part, (void*)pt, (void*)len, (void*)tab})
-      if (p) hipFree(p);
-  }
-};
-
-// Checks shared by the isolated attention entries; returns the longest route.
+// Checks shared by the isolated attention entries.
 static int attn_validate(rstr_pool* p, int32_t layer, int32_t batch, int32_t n_q, int32_t split, int32_t window,
-                         const float* q, const int32_t* pt, int32_t pps, const int32_t* len, int64_t* maxlen) {
+                         const float* q, const int32_t* pt, int32_t pps, const int32_t* len) {
   rstr_session* s = p->m->s;
   const auto& md = p->m->d;
   if (layer < 0 || layer >= md.n_layers) return fail(s, RSTR_E_INVALID, "layer out of range");
@@ -2005,42 +1996,13 @@ static int attn_validate(rstr_pool* p, int32_t layer, int32_t batch, int32_t n_q
   if (window < 0) return fail(s, RSTR_E_INVALID, "invalid window");
   if (!q || !pt || !len) return fail(s, RSTR_E_INVALID, "null attention input");
   int ps = p->page_size;
-  *maxlen = 0;
   for (int b = 0; b < batch; b++) {
     if (len[b] < 0 || (int64_t)len[b] > (int64_t)pps * ps) return fail(s, RSTR_E_INVALID, "length out of range");
     for (int i = 0; i < (len[b] + ps - 1) / ps; i++) {
       int32_t pg = pt[(int64_t)b * pps + i];
       if (pg < 0 || pg >= p->physical_pages) return fail(s, RSTR_E_INVALID, "page table entry out of range");
     }
-    *maxlen = std::max<int64_t>(*maxlen, len[b]);
   }
-  return RSTR_OK;
-}
-
-static int attn_prepare(rstr_pool* p, int32_t layer, int32_t batch, int32_t n_q, int32_t split,
-                        int32_t window, const float* q, const int32_t* pt, int32_t pps,
-                        const int32_t* len, AttnBufs& bf, AttnGeom& geo, int* max_items) {
-  rstr_session* s = p->m->s;
-  const auto& md = p->m->d;
-  int64_t maxlen = 0;
-  int rc = attn_validate(p, layer, batch, n_q, split, window, q, pt, pps, len, &maxlen);
-  if (rc) return rc;
-  int G = n_q / md.n_kv;
-  int hd = md.head_dim;
-  *max_items = (int)std::max<int64_t>(1, (int64_t)batch * md.n_kv * ((maxlen + split - 1) / split + 1));
-  HIPCHK(s, hipSetDevice(s->device));
-  HIPCHK(s, dmalloc(&bf.q, (size_t)batch * n_q * hd));
-  HIPCHK(s, dmalloc(&bf.out, (size_t)batch * n_q * hd));
-  HIPCHK(s, dmalloc(&bf.part, (size_t)*max_items * G * attn_part_floats(hd)));
-  HIPCHK(s, dmalloc(&bf.pt, (size_t)batch * pps));
-  HIPCHK(s, dmalloc(&bf.len, (size_t)batch));
-  geo = AttnGeom{batch, n_q, md.n_kv, hd, p->page_size, pps, split, window, 0.0f};
-  const size_t tabw = attn_tab_words(geo, *max_items);
-  if (tabw == 0) return fail(s, RSTR_E_INVALID, "unsupported attention geometry");
-  HIPCHK(s, dmalloc(&bf.tab, tabw));
-  HIPCHK(s, hipMemcpy(bf.q, q, sizeof(float) * batch * n_q * hd, hipMemcpyHostToDevice));
-  HIPCHK(s, hipMemcpy(bf.pt, pt, sizeof(int32_t) * batch * pps, hipMemcpyHostToDevice));
-  HIPCHK(s, hipMemcpy(bf.len, len, sizeof(int32_t) * batch, hipMemcpyHostToDevice));
   return RSTR_OK;
 }
 
@@ -2068,14 +2030,11 @@ struct AttnBlock {
   size_t o_q = 0, o_pt = 0, o_len = 0, o_out = 0, o_tab = 0, o_part = 0, total = 0;
 };
 static int attn_block(rstr_pool* p, int32_t layer, int32_t batch, int32_t n_q, int32_t split, int32_t window,
-                      float scale, const float* q, const int32_t* row_offsets, const int32_t* positions,
-                      const int32_t* page_table, int32_t pps, const int32_t* lengths, const int32_t* start_positions,
-                      float* out, AttnBlock& bk) {
+                      float scale, const float* q, const int32_t* page_table, int32_t pps, const int32_t* lengths,
+                      AttnBlock& bk) {
   rstr_session* s = p->m->s;
-  int rc = attn_check_rows(s, batch, row_offsets, positions, lengths, start_positions, out);
+  const int rc = attn_validate(p, layer, batch, n_q, split, window, q, page_table, pps, lengths);
   if (rc) return rc;
-  int64_t maxlen = 0;
-  if ((rc = attn_validate(p, layer, batch, n_q, split, window, q, page_table, pps, lengths, &maxlen))) return rc;
   const auto& md = p->m->d;
   const int hd = md.head_dim, G = n_q / md.n_kv;
   // exact item count: n_kv items per split of each lane's visible range
@@ -2123,8 +2082,9 @@ static hipError_t attn_launch(rstr_pool* p, int32_t layer, const AttnBlock& bk, 
 // The call's arrays are staged in pinned memory and sent with one copy into the
 // pool's device block, the output comes back the same way, and the host waits
 // once.  A device allocation per buffer and call, partials sized to the longest
-// route for every lane, and copies of pageable arrays took 6.5 ms around 0.24 ms
-// of kernels (128 Llama-3-8B lanes, contexts to 23 k).
+// route for every lane, and copies of pageable arrays took 4.9-6.5 ms (by box)
+// around 0.24 ms of kernels (128 Llama-3-8B lanes, contexts to 23 k), against
+// 0.49; a pool's first call, which allocates both blocks, takes 0.7.
 extern "C" int rstr_attention_run(rstr_pool* p, int32_t layer, int32_t batch, int32_t n_q, int32_t split,
                                   int32_t window, float scale, const float* q, const int32_t* row_offsets,
                                   const int32_t* positions, const int32_t* page_table, int32_t pps,
@@ -2132,9 +2092,9 @@ extern "C" int rstr_attention_run(rstr_pool* p, int32_t layer, int32_t batch, in
   if (!p) return fail(nullptr, RSTR_E_INVALID, "null pool");
   rstr_session* s = p->m->s;
   AttnBlock bk;
-  int rc = attn_block(p, layer, batch, n_q, split, window, scale, q, row_offsets, positions, page_table, pps, lengths,
-                      start_positions, out, bk);
+  int rc = attn_check_rows(s, batch, row_offsets, positions, lengths, start_positions, out);
   if (rc) return rc;
+  if ((rc = attn_block(p, layer, batch, n_q, split, window, scale, q, page_table, pps, lengths, bk))) return rc;
   hipStream_t st = s->stream;
   // grow what the pool keeps (nothing of an earlier call is still running), or
   // take memory for this call alone; what is kept is given back before more is
@@ -2214,9 +2174,9 @@ extern "C" int rstr_attention_run_static(rstr_pool* p, int32_t layer, int32_t ba
   if (!p) return fail(nullptr, RSTR_E_INVALID, "null pool");
   rstr_session* s = p->m->s;
   AttnBlock bk;
-  int rc = attn_block(p, layer, batch, n_q, split, window, scale, q, row_offsets, positions, page_table, pps, lengths,
-                      start_positions, out, bk);
+  int rc = attn_check_rows(s, batch, row_offsets, positions, lengths, start_positions, out);
   if (rc) return rc;
+  if ((rc = attn_block(p, layer, batch, n_q, split, window, scale, q, page_table, pps, lengths, bk))) return rc;
   if (bk.total > (size_t)RSTR_ATTN_STATIC_BYTES)
     return fail(s, RSTR_E_INVALID, "attention staging of " + std::to_string(bk.total) +
                                        " bytes exceeds the static staging maximum of " +
@@ -2240,24 +2200,34 @@ extern "C" int rstr_attention_bench(rstr_pool* p, int32_t layer, int32_t batch, 
   if (!p) return fail(nullptr, RSTR_E_INVALID, "null pool");
   rstr_session* s = p->m->s;
   if (iters <= 0) return fail(s, RSTR_E_INVALID, "iters must be positive");
-  AttnBufs bf;
-  AttnGeom geo;
-  int max_items = 0;
-  int rc = attn_prepare(p, layer, batch, n_q, split, window, q, page_table, pps, lengths, bf, geo, &max_items);
+  AttnBlock bk;
+  const int rc = attn_block(p, layer, batch, n_q, split, window, scale, q, page_table, pps, lengths, bk);
   if (rc) return rc;
-  geo.scale = scale;
+  struct Own {
+    char* dev = nullptr;
+    ~Own() {
+      if (dev) hipFree(dev);
+    }
+  } own;
+  HIPCHK(s, dev_alloc(&own.dev, bk.total));
+  char* base = own.dev;
+  HIPCHK(s, hipMemcpy(base + bk.o_q, q, bk.qb, hipMemcpyHostToDevice));
+  HIPCHK(s, hipMemcpy(base + bk.o_pt, page_table, bk.ptb, hipMemcpyHostToDevice));
+  HIPCHK(s, hipMemcpy(base + bk.o_len, lengths, bk.lb, hipMemcpyHostToDevice));
   hipStream_t st = s->stream;
-  int L = p->m->d.n_layers;
-  HIPCHK(s, launch_attn_lists(st, &geo, 1, bf.len, bf.tab, 0, max_items));
+  const int L = p->m->d.n_layers;
+  auto f = [&](size_t o) { return reinterpret_cast<float*>(base + o); };
+  auto i32 = [&](size_t o) { return reinterpret_cast<int32_t*>(base + o); };
+  HIPCHK(s, launch_attn_lists(st, &bk.geo, 1, i32(bk.o_len), i32(bk.o_tab), 0, bk.max_items));
   std::vector<hipEvent_t> ev(4 * iters);
   for (auto& e : ev) HIPCHK(s, hipEventCreate(&e));
   for (int i = 0; i < iters; i++) {
     HIPCHK(s, hipEventRecord(ev[4 * i], st));
-    HIPCHK(s, launch_attn_split(st, geo, bf.q, p->slabs[layer], p->slabs[L + layer], bf.pt, bf.tab, bf.part,
-                                max_items));
+    HIPCHK(s, launch_attn_split(st, bk.geo, f(bk.o_q), p->slabs[layer], p->slabs[L + layer], i32(bk.o_pt),
+                                i32(bk.o_tab), f(bk.o_part), bk.max_items));
     HIPCHK(s, hipEventRecord(ev[4 * i + 1], st));
     HIPCHK(s, hipEventRecord(ev[4 * i + 2], st));
-    HIPCHK(s, launch_attn_merge(st, geo, bf.len, bf.tab, bf.part, bf.out, nullptr));
+    HIPCHK(s, launch_attn_merge(st, bk.geo, i32(bk.o_len), i32(bk.o_tab), f(bk.o_part), f(bk.o_out), nullptr));
     HIPCHK(s, hipEventRecord(ev[4 * i + 3], st));
   }
   HIPCHK(s, hipStreamSynchronize(st));
