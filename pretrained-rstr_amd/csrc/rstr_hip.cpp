@@ -1110,6 +1110,10 @@ static int decoder_open(rstr_model* m, rstr_pool* p, int32_t batch, int32_t pps,
   const int s_d = std::max(d->s_o, d->s_down);
   int64_t max_pos_tokens = std::min<int64_t>((int64_t)pps * p->page_size, (int64_t)maxpos + 1);
   int64_t splits = (max_pos_tokens + split - 1) / split + 1;
+  // routes within one split have one item per kv head: 128 Llama-3-8B lanes of 300
+  // tokens at split 512 are 1024 items, not 2048, and stay with the few-item kernel,
+  // which needs no merge then (four layers 752 us a step against 771)
+  if (std::min<int64_t>((int64_t)pps * p->page_size, maxpos) <= split) splits = 1;
   d->max_items = (int)std::min<int64_t>((int64_t)batch * md.n_kv * splits, INT32_MAX / 4);
   int G = md.n_q / md.n_kv;
   d->off_slots = 0;
