@@ -2763,11 +2763,12 @@ __device__ __forceinline__ float qk_tree(float (&v)[G], int j) {
 // Bound by the chain of dependent loads in front (list entry, page ids and
 // query, rows: ~3 us) and the rows' own streaming.  Measured on MI355X, us a
 // launch, against a ring of 16-token chunks shared by the waves with a barrier
-// per chunk: five Qwen3-0.6B lanes (11.6 k tokens, 47 MB) 15.5 vs 22.7, seven
-// Llama-3-8B lanes 18 vs 28.9, one lane at split 64 7.5 vs 11.1, one
-// Gemma-3-270M lane of 64 tokens 10 vs 13.5.  On long lists the one-wave
-// kernel streams better (128 Llama-3-8B lanes 217 vs 274 us, 45 lanes 87 vs
-// 99), because a workgroup here has nothing in flight while it computes.
+// per chunk: five Qwen3-0.6B lanes (11.6 k tokens, 47 MB) 14.4 vs 22.7, seven
+// Llama-3-8B lanes 15.5 vs 28.9, one lane at split 64 7.8 vs 11.1, one
+// Gemma-3-270M lane of 64 tokens 10.4 vs 13.5.  On long lists at head dim 128
+// the one-wave kernel streams better (128 Llama-3-8B lanes 217 vs 274 us, 45
+// lanes 87 vs 99), because a workgroup here has nothing in flight while it
+// computes.
 // Every list position is static here, so no claims.
 //
 // QKV: the item's query comes from the qkv projection slices (QkvHeads; q is
@@ -3091,9 +3092,9 @@ __global__ __launch_bounds__(256, QKV ? (NC == 4 && G <= 4 && HD == 128 ? 3 : 1)
 // on this GPU: 34 cycles alone, 57 with four conversions), so a full 256-token
 // item is 8.7 k cycles of them per wave and about 6 k of conversions, slice
 // tree and exps.  Measured on MI355X (512 Llama-3-8B rows at position 3584,
-// 33.5 GFLOP a layer): 464 us a layer, against 1159 us for k_attn_split over
+// 33.5 GFLOP a layer): 457 us a layer, against 1159 us for k_attn_split over
 // the same rows as lanes (its fmas issue at 4.4 cycles for 64); 77 Qwen3-0.6B
-// rows over 1080 tokens 22.0 against 38.7 us.  Four waves over 64 pairs that
+// rows over 1080 tokens 22.3 against 38.7 us.  Four waves over 64 pairs that
 // share each K/V chunk through a barrier per chunk measured 500 and 55 us.
 typedef float f16v __attribute__((ext_vector_type(16)));
 
