@@ -158,6 +158,7 @@ struct HostRing {
 
 struct rstr_pool {
   rstr_model* m = nullptr;
+  int device = 0;
   int page_size = 0, physical_pages = 0;
   int64_t page_elems = 0;                 // page_size * n_kv * head_dim
   std::vector<uint16_t*> slabs;           // [K0..K{L-1}, V0..V{L-1}]
@@ -184,9 +185,14 @@ struct rstr_pool {
   size_t attn_dev_bytes = 0, attn_host_bytes = 0;
   bool attn_busy = false;  // a call uses them
 };
-// What a pool keeps for the isolated attention between calls, per buffer;
-// larger calls, and calls that find the buffers in use, allocate and free their own.
-static constexpr size_t kAttnKeep = (size_t)128 << 20;
+// What a pool keeps for the isolated attention between calls: a device block, and
+// pinned staging of arrays up to kAttnStage.  Calls with larger partials, and calls
+// that find the blocks in use, allocate and free a device block of their own; the
+// latter's arrays, and larger ones, go from and to the caller's memory: pinned memory costs 0.4 ms a MB when it is first
+// allocated and every byte another host copy, which is even with the runtime's own
+// staging at 12 MB (0.71 and 0.72 ms a call, at 3 MB 0.28 and 0.33, at 25 MB 1.62
+// and 1.43).
+static constexpr size_t kAttnKeep = (size_t)128 << 20, kAttnStage = (size_t)16 << 20;
 // The open pools; guards the list and every pool's attn_busy and idle blocks.
 static std::mutex g_pools_mu;
 static std::vector<rstr_pool*> g_pools;
@@ -207,7 +213,7 @@ bool release_kept_blocks() {
   std::lock_guard<std::mutex> lock(g_pools_mu);
   bool any = false;
   for (rstr_pool* p : g_pools)
-    if (!p->attn_busy && p->m->s->device == dev) any |= free_attn_blocks(p);
+    if (!p->attn_busy && p->device == dev) any |= free_attn_blocks(p);
   return any;
 }
 }  // namespace
@@ -721,6 +727,7 @@ extern "C" int rstr_pool_open(rstr_model* m, int32_t page_size, int32_t physical
   HIPCHK(s, hipSetDevice(s->device));
   auto p = std::make_unique<rstr_pool>();
   p->m = m;
+  p->device = s->device;
   p->page_size = page_size;
   p->physical_pages = physical_pages;
   p->page_elems = (int64_t)page_size * m->d.n_kv * m->d.head_dim;
@@ -2105,10 +2112,9 @@ extern "C" int rstr_attention_run(rstr_pool* p, int32_t layer, int32_t batch, in
   // asked for, so a call fits wherever it fits without it
   const size_t in_bytes = bk.o_out, host_bytes = std::max(in_bytes, bk.qb);
   struct Own {
-    void *dev = nullptr, *host = nullptr;
+    void* dev = nullptr;
     ~Own() {
       if (dev) hipFree(dev);
-      if (host) hipHostFree(host);
     }
   } own;
   struct Claim {
@@ -2126,7 +2132,7 @@ extern "C" int rstr_attention_run(rstr_pool* p, int32_t layer, int32_t batch, in
       kept.p = p;
     }
   }
-  void *dev = kept.p ? p->attn_dev : nullptr, *host = kept.p ? p->attn_host : nullptr;
+  void* dev = kept.p ? p->attn_dev : nullptr;
   if (!kept.p || bk.total > p->attn_dev_bytes) {
     if (kept.p && p->attn_dev) {
       hipFree(p->attn_dev);
@@ -2141,21 +2147,27 @@ extern "C" int rstr_attention_run(rstr_pool* p, int32_t layer, int32_t batch, in
       own.dev = dev;
     }
   }
-  if (!kept.p || host_bytes > p->attn_host_bytes) {
-    if (kept.p && p->attn_host) {
-      hipHostFree(p->attn_host);
-      p->attn_host = nullptr;
-      p->attn_host_bytes = 0;
-    }
-    HIPCHK(s, host_alloc(&host, host_bytes));
-    if (kept.p && host_bytes <= kAttnKeep) {
-      p->attn_host = host;
-      p->attn_host_bytes = host_bytes;
-    } else {
-      own.host = host;
-    }
+  const bool staged = kept.p && host_bytes <= kAttnStage;
+  if (staged && host_bytes > p->attn_host_bytes) {
+    if (p->attn_host) hipHostFree(p->attn_host);
+    p->attn_host = nullptr;
+    p->attn_host_bytes = 0;
+    HIPCHK(s, host_alloc(&p->attn_host, host_bytes));
+    p->attn_host_bytes = host_bytes;
   }
-  char *hb = static_cast<char*>(host), *db = static_cast<char*>(dev);
+  char* db = static_cast<char*>(dev);
+  if (!staged) {
+    HIPCHK(s, hipMemcpy(db + bk.o_q, q, bk.qb, hipMemcpyHostToDevice));
+    HIPCHK(s, hipMemcpy(db + bk.o_pt, page_table, bk.ptb, hipMemcpyHostToDevice));
+    HIPCHK(s, hipMemcpy(db + bk.o_len, lengths, bk.lb, hipMemcpyHostToDevice));
+    const hipError_t e = attn_launch(p, layer, bk, db);
+    const hipError_t e2 = hipStreamSynchronize(st);  // also on an error: the block is in use until here
+    HIPCHK(s, e);
+    HIPCHK(s, e2);
+    HIPCHK(s, hipMemcpy(out, db + bk.o_out, bk.qb, hipMemcpyDeviceToHost));
+    return RSTR_OK;
+  }
+  char* hb = static_cast<char*>(p->attn_host);
   std::memcpy(hb + bk.o_q, q, bk.qb);
   std::memcpy(hb + bk.o_pt, page_table, bk.ptb);
   std::memcpy(hb + bk.o_len, lengths, bk.lb);

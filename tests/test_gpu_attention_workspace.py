@@ -36,6 +36,28 @@ def test_calls_of_any_size_share_the_kept_blocks():
 
 
 @pytest.mark.gpu
+def test_large_arrays_go_without_the_staging_block():
+    """Page tables on both sides of the 16 MB that are staged, in turn on one pool;
+    the entries past a route are not read."""
+    print("case attention large arrays", flush=True)
+    cfg = dict(configs.TINY_QWEN, n_layers=1, n_q=8, n_kv=1, head_dim=128, vocab=512)
+    ps, pages, lanes = 16, 64, 9
+    rng = np.random.default_rng(6)
+    with hip.Session(0) as s:
+        p = hip.Pool(hip.Model(s, cfg, seed=1), ps, pages)
+        p.fill_synthetic(np.arange(pages), seed=3)
+        q = rng.standard_normal((lanes, 8, 128)).astype(np.float32)
+        table = np.stack([rng.permutation(pages) for _ in range(lanes)]).astype(np.int32)
+        lengths = rng.integers(1, pages * ps + 1, lanes).astype(np.int32)
+        want = p.attention(0, q, table, lengths, split=64, static=True)
+        for width in (pages, 600_000, 400_000, pages, 465_000):
+            wide = np.full((lanes, width), -1, np.int32)
+            wide[:, :pages] = table
+            got = p.attention(0, q, wide, lengths, split=64)
+            assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), width
+
+
+@pytest.mark.gpu
 def test_a_call_beside_another_takes_its_own_blocks():
     print("case attention beside attention", flush=True)
     cfg = dict(configs.TINY_QWEN, n_layers=1, n_q=8, n_kv=1, head_dim=128, vocab=512)
